@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(BLOCK) k_advect(TB t, const double *__restrict
 // T u H1, then advect_value for T.  out = result, or (RK_AVG) out = (out +
 // result) / 2.  The loads a node needs (its record, slot and vn, and the
 // value being averaged) are issued before the first barrier.
-template <int D, bool RK_AVG>
+template <int D, bool RK_AVG, bool WT>
 __global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_per_eu(CASL_TILE_WAVES_F64)))
     k_tile_advect(TileArgs<double> A, const double *__restrict__ vn, double dt) {
   constexpr int DMAX = TileLimits<D>::DMAX;
@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_pe
   TileCtx<D> c;
   c.load(A, tile);
   const int s = c.s, nT = c.nT, hb = c.hb, nH = c.nH, nH1 = c.nH1;
-  const bool ufast = A.geom.pow2 != 0 && A.geom.cubic != 0;
+  const bool ufast = A.geom.template uni_fast<WT>();
   RecRegs trec[KT];
   int tslot[KT];
 #pragma unroll
@@ -75,12 +75,12 @@ __global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_pe
 #pragma unroll
   for (int k = 0; k < KT; ++k) {
     const int i = int(threadIdx.x) + k * TILE_BLOCK_F64;
-    if (i < nT) tile_pass_a<D, double>(A, c, ufast, trec[k], tslot[k], i, phis, dds);
+    if (i < nT) tile_pass_a<D, double, WT>(A, c, ufast, trec[k], tslot[k], i, phis, dds);
   }
   for (int i = nT + int(threadIdx.x); i < nT + nH1; i += TILE_BLOCK_F64) {
     RecRegs r;
     const int js = fetch_record<D>(A, c, i, r);
-    tile_pass_a<D, double>(A, c, ufast, r, js, i, phis, dds);
+    tile_pass_a<D, double, WT>(A, c, ufast, r, js, i, phis, dds);
   }
   __syncthreads();
 #pragma unroll
@@ -90,18 +90,18 @@ __global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_pe
     int j = tslot[k];
     double r;
     if (ufast && c.uniform(i)) {
-      UniStencil<D, double> st;
+      UniStencil<D, double, WT> st;
       j = st.load(trec[k].w, A.geom);
       r = advect_value<D>(st, j, 0, vn[s + j], dt, phis, dds, DMAX);
     } else {
       const TileRec rec = record_at<D>(c, i, trec[k], j);
       const uint8_t w = uint8_t((rec.geo >> 24) & 63u);
       if (!(rec.geo & GEO_IRREGULAR)) {
-        RegStencil<D, double> st;
+        RegStencil<D, double, WT> st;
         st.load(rec, A.geom);
         r = advect_value<D>(st, j, w, vn[s + j], dt, phis, dds, DMAX);
       } else {
-        HangStencil<D, double> st;
+        HangStencil<D, double, WT> st;
         st.load(rec, c.ext_of(A.ext, i), A.geom);
         r = advect_value<D>(st, j, w, vn[s + j], dt, phis, dds, DMAX);
       }
@@ -146,15 +146,22 @@ void run_advect(casl_stencil *st, double *phi, const double *vn, const double *v
     st->phi0.ensure(N);
     TileArgs<double> ta = tile_args<double>(st);
     const dim3 g(unsigned(st->n_tiles)), b(TILE_BLOCK_F64);
+    const bool wt = st->weighted_tiles();
     ta.phin = phi;
     ta.out = st->phi0.p;
     prof_begin("k_tile_advect", s);
-    hipLaunchKernelGGL((k_tile_advect<D, false>), g, b, 0, s, ta, vn, dt);
+    if (wt)
+      hipLaunchKernelGGL((k_tile_advect<D, false, true>), g, b, 0, s, ta, vn, dt);
+    else
+      hipLaunchKernelGGL((k_tile_advect<D, false, false>), g, b, 0, s, ta, vn, dt);
     prof_end("k_tile_advect", s);
     ta.phin = st->phi0.p;
     ta.out = phi;
     prof_begin("k_tile_advect", s);
-    hipLaunchKernelGGL((k_tile_advect<D, true>), g, b, 0, s, ta, vnp1 ? vnp1 : vn, dt);
+    if (wt)
+      hipLaunchKernelGGL((k_tile_advect<D, true, true>), g, b, 0, s, ta, vnp1 ? vnp1 : vn, dt);
+    else
+      hipLaunchKernelGGL((k_tile_advect<D, true, false>), g, b, 0, s, ta, vnp1 ? vnp1 : vn, dt);
     prof_end("k_tile_advect", s);
     HIP_CHECK(hipGetLastError());
     return;

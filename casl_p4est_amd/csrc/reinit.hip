@@ -24,6 +24,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -178,6 +179,10 @@ dev::TileArgs<R> tile_args(const casl_stencil *st) {
     ta.geom.base_bits[a] = exp_word(ta.geom.base[a]);
     ta.geom.inv_bits[a] = exp_word(ta.geom.inv_base[a]);
   }
+  // one product serves every regular face (2D: one transverse extent)
+  const R wgt = st->dim == 2 ? ta.geom.base[0] : ta.geom.base[0] * ta.geom.base[0];
+  ta.geom.wgt = wgt;
+  ta.geom.inv_wgt = R(1) / wgt;
   ta.geom.cubic = 1;
   for (int a = 1; a < st->dim; ++a) ta.geom.cubic &= int(st->geom_base[a] == st->geom_base[0]);
   ta.geom.d_pack = 0;
@@ -239,6 +244,20 @@ ReinitSizes reinit_sizes(size_t N, bool so, bool tiled) {
   return z;
 }
 
+// fn(wt): wt is true for FP64 on a geometry that is not dyadic, where the
+// kernels keep the weighted form of regular faces; the mixed path's FP32
+// stages (and its prep) do not need it.
+template <class R, class Fn>
+void with_weights(bool weighted, Fn &&fn) {
+  if constexpr (sizeof(R) == 8) {
+    if (weighted) {
+      fn(std::true_type{});
+      return;
+    }
+  }
+  fn(std::false_type{});
+}
+
 // Every scratch buffer a reinitialization call of this kind uses, allocated
 // up front in the stencil (a recorded graph must not allocate).
 template <int D, class R>
@@ -280,7 +299,7 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
   const bool so = order_space > 1;
   const unsigned grid = grid_for(N);
 
-  const bool tiled = st->use_tiles(sizeof(R) == 8);
+  const bool tiled = st->use_tiles(sizeof(R) == 8), wt_tiles = st->weighted_tiles();
   HIP_CHECK(hipMemcpyAsync(B.phi0, phi, sizeof(double) * N, hipMemcpyDeviceToDevice, s));
   if (so && !tiled) {
     prof_begin("k_dd", s);
@@ -304,12 +323,11 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
     tp.phin = B.phi0;
     const dim3 g(unsigned(st->n_tiles)), b(TILE_BLOCK_F64);
     prof_begin("k_tile_prep", s);
-    if (so)
-      hipLaunchKernelGGL((k_tile_prep<D, R, true>), g, b, 0, s, tp, mask, lim_low, lim_high, st->zdt, B.flags,
-                         sfix);
-    else
-      hipLaunchKernelGGL((k_tile_prep<D, R, false>), g, b, 0, s, tp, mask, lim_low, lim_high, st->zdt, B.flags,
-                         sfix);
+    auto prep = [&](auto second, auto wt) {
+      hipLaunchKernelGGL((k_tile_prep<D, R, decltype(second)::value, decltype(wt)::value>), g, b, 0, s, tp, mask,
+                         lim_low, lim_high, st->zdt, B.flags, sfix);
+    };
+    with_weights<R>(wt_tiles, [&](auto wt) { so ? prep(std::true_type{}, wt) : prep(std::false_type{}, wt); });
     prof_end("k_tile_prep", s);
   } else {
     prof_begin("k_prep", s);
@@ -367,17 +385,16 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
     ta.out = out;
     const dim3 g(unsigned(st->n_tiles)), b(stage_block<R>());
     prof_begin("k_tile_stage", s);
-    if (so) {
-      if (avg)
-        hipLaunchKernelGGL((k_tile_stage<D, R, true, true>), g, b, 0, s, ta);
+    auto launch = [&](auto second, auto rk, auto wt) {
+      hipLaunchKernelGGL(
+          (k_tile_stage<D, R, decltype(second)::value, decltype(rk)::value, decltype(wt)::value>), g, b, 0, s, ta);
+    };
+    with_weights<R>(wt_tiles, [&](auto wt) {
+      if (so)
+        avg ? launch(std::true_type{}, std::true_type{}, wt) : launch(std::true_type{}, std::false_type{}, wt);
       else
-        hipLaunchKernelGGL((k_tile_stage<D, R, true, false>), g, b, 0, s, ta);
-    } else {
-      if (avg)
-        hipLaunchKernelGGL((k_tile_stage<D, R, false, true>), g, b, 0, s, ta);
-      else
-        hipLaunchKernelGGL((k_tile_stage<D, R, false, false>), g, b, 0, s, ta);
-    }
+        avg ? launch(std::false_type{}, std::true_type{}, wt) : launch(std::false_type{}, std::false_type{}, wt);
+    });
     prof_end("k_tile_stage", s);
   };
   for (int it = 0; it < n_iter; ++it) {
@@ -538,6 +555,7 @@ void upload_tile_host(const TileHost &H, int64_t n_nodes, casl_stencil *st) {
   st->n_records = int64_t(H.rec.size()) + int64_t(H.urec_start.back());
   st->n_uniform = int64_t(H.urec_start.back());
   st->n_irregular = H.n_irregular;
+  st->regular_weights = H.regular_weights;
   for (int a = 0; a < 3; ++a) {
     st->geom_base[a] = H.size[a];
     st->geom_unit[a] = H.size[a] * std::ldexp(1.0, -H.lmax);
@@ -801,6 +819,10 @@ int casl_stencil_tile_check(const casl_stencil_t *st, const casl_flat_stencil *t
     if (st->n_tiles != nt || st->n_halo != int64_t(H.halo_idx.size()) ||
         st->n_records != int64_t(H.rec.size()) + int64_t(H.urec_start.back()) || st->n_irregular != H.n_irregular) {
       set_error("tiled encodings differ in their counts");
+      return;
+    }
+    if (st->regular_weights != H.regular_weights) {
+      set_error("tiled encodings differ in their regular weights");
       return;
     }
     for (int a = 0; a < 3; ++a)

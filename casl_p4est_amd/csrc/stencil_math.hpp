@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
+#include "known_div.hpp"
+
 namespace casl {
 namespace dev {
 
@@ -23,6 +25,7 @@ struct Tables {
   static constexpr bool FASTDIV = false;  // see second_difference
   static constexpr bool SLOTS = false;    // see the hanging-face functions below
   static constexpr bool UNIFORM = false;  // see second_difference
+  static constexpr bool WEIGHTED = false; // see face_linear
   static constexpr int F = 2 * D;
   static constexpr int C = 1 << (D - 1);
   static constexpr int T = 2 * (D - 1);
@@ -161,11 +164,19 @@ __device__ __forceinline__ R div_dsum(const TB &t, R x, int a, int64_t n) {
 // correct_naive_second_derivatives is 0 and every quadratic correction is
 // 0.5*0*f'' = 0.  The REGULAR shortcuts therefore return the same values as
 // the full expressions for finite inputs (at most the sign of a zero differs).
+//
+// TB::WEIGHTED marks FP64 stencils of cubic cells whose edge is not a power of
+// two: (f_c w)/w then rounds twice and differs from f_c.  w is the edge (2D)
+// or its rounded square (3D) times a power of two, so the value depends on
+// the geometry alone and reg_value(f_c) gives it.
 template <int D, class R, class G, class TB>
 __device__ __forceinline__ R face_linear(const TB &t, int f, int64_t n, const G *__restrict__ g) {
   const R d_m0 = R(t.dt(f, 0, n)), d_p0 = R(t.dt(f, 1, n));
   if constexpr (TB::REGULAR) {
-    return R(g[t.idx(f, 0, n)]);
+    if constexpr (TB::WEIGHTED)
+      return t.reg_value(R(g[t.idx(f, 0, n)]));
+    else
+      return R(g[t.idx(f, 0, n)]);
   } else if constexpr (D == 2) {
     const R w_mm = d_p0;
     const R w_pm = d_m0;
@@ -216,8 +227,21 @@ __device__ __forceinline__ R central_second_derivative(R fp, R f0, R fm, R dp, R
 // in FP32.
 template <class R, class TB>
 __device__ __forceinline__ R second_difference(const TB &t, int a, R fp, R f0, R fm, int64_t n) {
-  if constexpr (TB::UNIFORM) return ((fp - f0) + (fm - f0)) * t.iq2[a];
   const int fpp = 2 * a + 1, fmm = 2 * a;
+  if constexpr (TB::WEIGHTED) {
+    // known reciprocals of the arms; equal arms: d_p + d_m = 2 d_p
+    if (t.nowall) {
+      const R x = (div_known(fp - f0, t.dist[fpp], t.iq[fpp]) + div_known(fm - f0, t.dist[fmm], t.iq[fmm])) * R(2.);
+      if constexpr (TB::UNIFORM) {
+        return div_known(x, R(2.) * t.dist[fpp], R(0.5) * t.iq[fpp]);
+      } else {
+        return t.dist[fpp] == t.dist[fmm] ? div_known(x, R(2.) * t.dist[fpp], R(0.5) * t.iq[fpp])
+                                          : x / (t.dist[fpp] + t.dist[fmm]);
+      }
+    }
+    return central_second_derivative(fp, f0, fm, R(t.d(fpp, n)), R(t.d(fmm, n)));
+  }
+  if constexpr (TB::UNIFORM) return ((fp - f0) + (fm - f0)) * t.iq2[a];
   if constexpr (TB::FASTDIV) {
     if (t.fast) {
       const R x = qfma(fp - f0, t.iq[fpp], (fm - f0) * t.iq[fmm]) * R(2.);
@@ -409,7 +433,10 @@ template <int D, class R, bool CORR, class G, class TB>
 __device__ __forceinline__ void hang_face_values(const TB &t, const G *__restrict__ g, R *fnb, const R *dd, R *vq) {
   constexpr int F = 2 * D;
 #pragma unroll
-  for (int f = 0; f < F; ++f) fnb[f] = R(g[t.id[f]]);
+  for (int f = 0; f < F; ++f) {
+    fnb[f] = R(g[t.id[f]]);
+    if constexpr (TB::WEIGHTED) fnb[f] = t.reg_value(fnb[f]);
+  }
 #pragma unroll
   for (int q = 0; q < TB::NH; ++q) {
     const int f = t.hface(q);
@@ -429,7 +456,10 @@ template <int D, class R, class G, class TB>
 __device__ __forceinline__ void hang_face_values_dd(const TB &t, const G *__restrict__ dd, int64_t stride, R *out) {
   constexpr int F = 2 * D;
 #pragma unroll
-  for (int f = 0; f < F; ++f) out[f] = R(dd[int64_t(f >> 1) * stride + t.id[f]]);
+  for (int f = 0; f < F; ++f) {
+    out[f] = R(dd[int64_t(f >> 1) * stride + t.id[f]]);
+    if constexpr (TB::WEIGHTED) out[f] = t.reg_value(out[f]);
+  }
 #pragma unroll
   for (int q = 0; q < TB::NH; ++q) {
     const int f = t.hface(q);

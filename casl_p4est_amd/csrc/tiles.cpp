@@ -23,6 +23,7 @@ struct Builder {
   double base[3] = {0, 0, 0};  // coarsest arm-cell size per axis
   int Lrel = 0;                // finest relative level
   double unit[3] = {0, 0, 0};
+  mutable std::atomic<bool> regular_weights{true};
 
   explicit Builder(const casl_flat_stencil &t) : tab(t), N(t.n_nodes) {}
 
@@ -104,6 +105,12 @@ struct Builder {
     });
     Lrel = lr.load();
     for (int a = 0; a < D; ++a) unit[a] = base[a] * std::ldexp(1.0, -Lrel);
+  }
+
+  // v is 0 or base times a power of two
+  static bool scale_multiple(double b, double v) {
+    int eb = 0, ev = 0;
+    return v == 0.0 || std::frexp(b, &eb) == std::frexp(v, &ev);
   }
 
   uint16_t units(int ax, double v) const {
@@ -262,6 +269,12 @@ struct Builder {
             if (local(t, nbr(f, c, n)) != r.idx[f]) throw std::runtime_error("tile record: corner mismatch");
           }
         if (nz != 1) throw std::runtime_error("tile record: hanging face not in the extension");
+        for (int k = 0; k < 2 * (D - 1); ++k) {
+          int ax, t2;
+          transverse(f >> 1, ax, t2);
+          if (k >= 2) ax = t2;
+          if (!scale_multiple(base[ax], dt(f, k, n))) regular_weights = false;
+        }
         continue;
       }
       int t1, t2;
@@ -409,6 +422,7 @@ struct Builder {
         H.nuni.push_back(uint32_t(t.n_tuni) | (uint32_t(t.n_h1uni) << 16));
       }
     H.n_irregular = int64_t(n_ext);
+    H.regular_weights = regular_weights;
     if (H.halo_idx.size() >= size_t(INT32_MAX) || H.rec.size() >= size_t(INT32_MAX) ||
         H.urec.size() / UW >= size_t(INT32_MAX))
       throw std::runtime_error("tile tables too large for int32 offsets");

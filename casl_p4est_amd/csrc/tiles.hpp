@@ -40,10 +40,12 @@
 #include "../../include/casl_reinit.h"
 
 // functions shared by the host builder (g++) and the device kernels (hipcc)
+#ifndef CASL_HD
 #ifdef __HIPCC__
 #define CASL_HD __host__ __device__
 #else
 #define CASL_HD
+#endif
 #endif
 
 namespace casl {
@@ -203,6 +205,8 @@ struct TileHost {
   std::vector<int32_t> ext_start;   // [ntiles + 1] first extension record of each tile
   std::vector<uint32_t> nreg;       // [ntiles] regular records of T (low 16 bits) and of H1 (high 16 bits)
   int64_t n_irregular = 0;
+  // every regular face's nonzero transverse offsets are base * 2^-l for some l
+  bool regular_weights = true;
 };
 
 // Builds the tiled encoding of a flattened stencil; throws std::runtime_error

@@ -27,6 +27,15 @@ struct TileGeom {
   // pow2 only: the bit pattern (FP32) or high word (FP64) of base and 1/base,
   // whose exponent field a level nibble moves down or up
   uint32_t base_bits[3], inv_bits[3];
+  // WEIGHTED stencils (FP64, cubic cells, base not a power of two): the one
+  // significand of all corner weights, base in 2D and RN(base^2) in 3D, and
+  // its correctly rounded reciprocal
+  R wgt, inv_wgt;
+  // uniform records decode as UniStencil
+  template <bool WT>
+  __device__ __forceinline__ bool uni_fast() const {
+    return WT || (pow2 != 0 && cubic != 0);
+  }
 };
 
 __device__ __forceinline__ double pow2neg(double, int l) { return __longlong_as_double((1023ll - l) << 52); }
@@ -43,10 +52,10 @@ __device__ __forceinline__ uint32_t level_exp(double, uint32_t geo, int f) { ret
 __device__ __forceinline__ float from_exp_bits(float, uint32_t b) { return __uint_as_float(b); }
 __device__ __forceinline__ double from_exp_bits(double, uint32_t b) { return __hiloint2double(int(b), 0); }
 
-template <int D, class R>
+template <int D, class R, bool WT = false>
 __device__ __forceinline__ void decode_dist(uint32_t geo, const TileGeom<R> &g, R *dist, R *q, R *iq) {
   constexpr int F = 2 * D;
-  if (sizeof(R) == 8 && g.pow2) {
+  if (!WT && sizeof(R) == 8 && g.pow2) {
     // FP64: base * 2^-l and 2^l / base by exponent arithmetic on the high
     // word (same values, fewer two-word operations); FP32 keeps the
     // multiplications, which measured faster there
@@ -79,8 +88,26 @@ __device__ __forceinline__ void decode_dist(uint32_t geo, const TileGeom<R> &g, 
 // wall arm, so every face distance d is a power of two and x / d == x * iq
 // exactly (both are the correctly rounded value of the same real number);
 // FASTDIV lets the stencil arithmetic use that.
-template <int D, class R>
-struct DecodedDist {
+// WT: FP64 on cubic cells whose edge is not a power of two (see face_linear's
+// WEIGHTED); q and dist are base * 2^-l and iq = RN(1 / q) = RN(1 / base) * 2^l.
+template <class R, bool WT>
+struct RegWeight {
+  static constexpr bool WEIGHTED = false;
+  __device__ __forceinline__ void set_weight(const TileGeom<R> &) {}
+};
+template <class R>
+struct RegWeight<R, true> {
+  static constexpr bool WEIGHTED = true;
+  R wgt, inv_wgt;
+  __device__ __forceinline__ void set_weight(const TileGeom<R> &g) {
+    wgt = g.wgt;
+    inv_wgt = g.inv_wgt;
+  }
+  __device__ __forceinline__ R reg_value(R x) const { return weighted_by(x, wgt, inv_wgt); }
+};
+
+template <int D, class R, bool WT = false>
+struct DecodedDist : RegWeight<R, WT> {
   static constexpr bool FASTDIV = true;
   static constexpr bool SLOTS = false;
   static constexpr bool UNIFORM = false;
@@ -88,17 +115,19 @@ struct DecodedDist {
   R dist[F];
   R q[F];
   R iq[F];
-  bool fast;
+  bool fast, nowall;
   __device__ __forceinline__ R d(int f, int64_t) const { return dist[f]; }
   __device__ __forceinline__ void decode(uint32_t geo, const TileGeom<R> &g) {
-    decode_dist<D, R>(geo, g, dist, q, iq);
-    fast = g.pow2 && ((geo >> 24) & 63u) == 0u;
+    decode_dist<D, R, WT>(geo, g, dist, q, iq);
+    nowall = ((geo >> 24) & 63u) == 0u;
+    fast = !WT && g.pow2 && nowall;
+    this->set_weight(g);
   }
 };
 
 // Stencil of a regular node (no hanging arm): one LDS-local corner per face.
-template <int D, class R>
-struct RegStencil : DecodedDist<D, R> {
+template <int D, class R, bool WT = false>
+struct RegStencil : DecodedDist<D, R, WT> {
   static constexpr bool REGULAR = true;
   static constexpr int F = 2 * D;
   uint16_t id[F];
@@ -112,19 +141,20 @@ struct RegStencil : DecodedDist<D, R> {
   }
 };
 
-// Stencil of a uniform node on a dyadic geometry of cubic cells (every arm
-// cell a power of two, one scale on every axis; the kernels take this
-// accessor only when TileGeom::pow2 and cubic, other geometries decode these
-// records as RegStencil): one corner per face, all arms q = base * 2^-level
+// Stencil of a uniform node on a geometry of cubic cells (one scale on every
+// axis) that is dyadic (every arm cell a power of two) or WT; the kernels take
+// this accessor only then, other geometries decode these records as
+// RegStencil: one corner per face, all arms q = base * 2^-level
 // long, no wall.  The per-face arrays hold the same value so the shared
 // stencil code reads them as it reads a RegStencil's.
-template <int D, class R>
-struct UniStencil {
+template <int D, class R, bool WT = false>
+struct UniStencil : RegWeight<R, WT> {
   static constexpr bool REGULAR = true;
   static constexpr bool FASTDIV = true;
   static constexpr bool SLOTS = false;
   static constexpr bool UNIFORM = true;
-  static constexpr bool fast = true;
+  static constexpr bool fast = !WT;
+  static constexpr bool nowall = true;
   static constexpr int F = 2 * D;
   uint16_t id[F];
   R dist[F], q[F], iq[F];
@@ -146,6 +176,7 @@ struct UniStencil {
     }
 #pragma unroll
     for (int a = 0; a < D; ++a) iq2[a] = iqq2;
+    this->set_weight(g);
     return slot;
   }
 };
@@ -167,8 +198,8 @@ __device__ __forceinline__ TileRec uni_as_rec(const uint32_t *w, int &slot) {
 // for the faces that hang (at most D - 1) the extension record's corners and
 // transverse offsets.  idx / dt serve any face (the per-face functions); the
 // hanging-face functions of stencil_math.hpp use hface / hidx / hdt.
-template <int D, class R>
-struct HangStencil : DecodedDist<D, R> {
+template <int D, class R, bool WT = false>
+struct HangStencil : DecodedDist<D, R, WT> {
   static constexpr bool REGULAR = false;
   static constexpr bool SLOTS = true;
   static constexpr int F = 2 * D, C = 1 << (D - 1);
@@ -277,7 +308,7 @@ struct HangStencil : DecodedDist<D, R> {
       e[2 * i] = v.x;
       e[2 * i + 1] = v.y;
     }
-    pow2 = g.pow2 != 0;
+    pow2 = !WT && g.pow2 != 0;
     geo = rec.geo;
 #pragma unroll
     for (int k = 0; k < D; ++k) {
@@ -417,9 +448,9 @@ __device__ __forceinline__ int slot_at(const TileCtx<D> &c, int i, const RecRegs
 }
 
 // Pass A (laplace) of the record at position i into dds[a * DMAX + slot].
-// Uniform records on a dyadic geometry (ufast) take UniStencil, the others
-// the general decoding.
-template <int D, class R>
+// Uniform records where UniStencil holds (ufast: see TileGeom::uni_fast) take
+// it, the others the general decoding.
+template <int D, class R, bool WT = false>
 __device__ __forceinline__ void tile_pass_a(const TileArgs<R> &A, const TileCtx<D> &c, bool ufast, const RecRegs &r,
                                             int fetched_slot, int i, const R *__restrict__ phis,
                                             R *__restrict__ dds) {
@@ -427,17 +458,17 @@ __device__ __forceinline__ void tile_pass_a(const TileArgs<R> &A, const TileCtx<
   R f000, fnb[2 * D], dd[D];
   int j = fetched_slot;
   if (ufast && c.uniform(i)) {
-    UniStencil<D, R> st;
+    UniStencil<D, R, WT> st;
     j = st.load(r.w, A.geom);
     laplace<D, R>(st, j, phis, f000, fnb, dd);
   } else {
     const TileRec rec = record_at<D>(c, i, r, j);
     if (!(rec.geo & GEO_IRREGULAR)) {
-      RegStencil<D, R> st;
+      RegStencil<D, R, WT> st;
       st.load(rec, A.geom);
       laplace<D, R>(st, j, phis, f000, fnb, dd);
     } else {
-      HangStencil<D, R> st;
+      HangStencil<D, R, WT> st;
       st.load(rec, c.ext_of(A.ext, i), A.geom);
       laplace<D, R>(st, j, phis, f000, fnb, dd);
     }
@@ -485,7 +516,7 @@ constexpr int stage_block() {
 // arrays phis[LMAX] and dds[D * DMAX].  It reads and writes global memory and
 // the LDS arrays only; a caller running several tiles in a row separates them
 // with a barrier (the next tile overwrites the LDS arrays).
-template <int D, class R, bool SECOND_ORDER, bool RK_AVG, int BLOCK>
+template <int D, class R, bool SECOND_ORDER, bool RK_AVG, int BLOCK, bool WT = false>
 __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__restrict__ phis,
                                            R *__restrict__ dds) {
   constexpr int DMAX = TileLimits<D>::DMAX;
@@ -494,7 +525,7 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
   TileCtx<D> c;
   c.load(A, tile);
   const int s = c.s, nT = c.nT, hb = c.hb, nH = c.nH, nH1 = c.nH1;
-  const bool ufast = A.geom.pow2 != 0 && A.geom.cubic != 0;
+  const bool ufast = A.geom.template uni_fast<WT>();
   RecRegs trec[KT];
   uint32_t tsf[KT];  // LDS slot of a non-uniform record (low 16 bits) and flags (high 16 bits)
   // the phi_n averaged with in the second RK2 stage: loaded before the first
@@ -574,17 +605,17 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
 #pragma unroll
     for (int k = 0; k < KT; ++k) {
       const int i = int(threadIdx.x) + k * BLOCK;
-      if (i < nT) tile_pass_a<D, R>(A, c, ufast, trec[k], int(tsf[k] & 0xffffu), i, phis, dds);
+      if (i < nT) tile_pass_a<D, R, WT>(A, c, ufast, trec[k], int(tsf[k] & 0xffffu), i, phis, dds);
     }
 #pragma unroll
     for (int k = 0; k < K1; ++k) {
       const int i = nT + int(threadIdx.x) + k * BLOCK;
-      if (i < nT + nH1) tile_pass_a<D, R>(A, c, ufast, hrec[k], hslot[k], i, phis, dds);
+      if (i < nT + nH1) tile_pass_a<D, R, WT>(A, c, ufast, hrec[k], hslot[k], i, phis, dds);
     }
     for (int i = nT + int(threadIdx.x) + K1 * BLOCK; i < nT + nH1; i += BLOCK) {
       RecRegs r;
       const int js = fetch_record<D>(A, c, i, r);
-      tile_pass_a<D, R>(A, c, ufast, r, js, i, phis, dds);
+      tile_pass_a<D, R, WT>(A, c, ufast, r, js, i, phis, dds);
     }
     __syncthreads();
   }
@@ -608,9 +639,10 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
     const int i = int(threadIdx.x) + k * BLOCK;
     if (!(ufast && i < c.nTu)) continue;
     const uint16_t fl = uint16_t(tsf[k] >> 16);
-    UniStencil<D, R> st;
+    using ST = UniStencil<D, R, WT>;
+    ST st;
     const int j = st.load(trec[k].w, A.geom);
-    const R r = stage_value<D, R, SECOND_ORDER, UniStencil<D, R>, true>(st, j, fl, 0, A.sfix + (s + i), A.N,
+    const R r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, 0, A.sfix + (s + i), A.N,
                                                                           A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
     store(k, int64_t(s) + j, r);
   }
@@ -624,14 +656,16 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
     const TileRec rec = record_at<D>(c, i, trec[k], j);
     const uint8_t w = uint8_t((rec.geo >> 24) & 63u);
     if (!(rec.geo & GEO_IRREGULAR)) {
-      RegStencil<D, R> st;
+      using ST = RegStencil<D, R, WT>;
+      ST st;
       st.load(rec, A.geom);
-      r = stage_value<D, R, SECOND_ORDER, RegStencil<D, R>, true>(st, j, fl, w, A.sfix + (s + i), A.N,
+      r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, A.sfix + (s + i), A.N,
                                                                    A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
     } else {
-      HangStencil<D, R> st;
+      using ST = HangStencil<D, R, WT>;
+      ST st;
       st.load(rec, c.ext_of(A.ext, i), A.geom);
-      r = stage_value<D, R, SECOND_ORDER, HangStencil<D, R>, true>(st, j, fl, w, A.sfix + (s + i), A.N,
+      r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, A.sfix + (s + i), A.N,
                                                                     A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
     }
     store(k, int64_t(s) + j, r);
@@ -642,7 +676,7 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
 // pass A of phi_0 for T u H1 (second order), then flags and s_fix of the
 // tile's nodes, written in record order (tile start + record position), the
 // order the stage body reads them in.  A.phin is phi_0.
-template <int D, class S, bool SECOND_ORDER, int BLOCK>
+template <int D, class S, bool SECOND_ORDER, int BLOCK, bool WT = false>
 __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, double *__restrict__ phis,
                                           double *__restrict__ dds, const uint8_t *__restrict__ mask,
                                           double lim_low, double lim_high, double zdt,
@@ -651,7 +685,7 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
   TileCtx<D> c;
   c.load(A, tile);
   const int s = c.s, nT = c.nT, hb = c.hb, nH = c.nH, nH1 = c.nH1;
-  const bool ufast = A.geom.pow2 != 0 && A.geom.cubic != 0;
+  const bool ufast = A.geom.template uni_fast<WT>();
   for (int j = threadIdx.x; j < nT; j += BLOCK) phis[j] = A.phin[s + j];
   for (int j = threadIdx.x; j < nH; j += BLOCK) phis[nT + j] = A.phin[A.halo[hb + j]];
   __syncthreads();
@@ -659,7 +693,7 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
     for (int i = int(threadIdx.x); i < nT + nH1; i += BLOCK) {
       RecRegs r;
       const int js = fetch_record<D>(A, c, i, r);
-      tile_pass_a<D, double>(A, c, ufast, r, js, i, phis, dds);
+      tile_pass_a<D, double, WT>(A, c, ufast, r, js, i, phis, dds);
     }
     __syncthreads();
   }
@@ -668,23 +702,26 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
     int j = fetch_record<D>(A, c, i, r);
     uint16_t fl;
     if (ufast && c.uniform(i)) {
-      UniStencil<D, double> st;
+      using ST = UniStencil<D, double, WT>;
+      ST st;
       j = st.load(r.w, A.geom);
       const bool masked = mask && mask[s + j] == 0;
-      fl = prep_value<D, S, UniStencil<D, double>, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low, lim_high,
+      fl = prep_value<D, S, ST, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low, lim_high,
                                                                   zdt, SECOND_ORDER, sfix + (s + i), A.N);
     } else {
       const TileRec rec = record_at<D>(c, i, r, j);
       const bool masked = mask && mask[s + j] == 0;
       if (!(rec.geo & GEO_IRREGULAR)) {
-        RegStencil<D, double> st;
+        using ST = RegStencil<D, double, WT>;
+        ST st;
         st.load(rec, A.geom);
-        fl = prep_value<D, S, RegStencil<D, double>, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low,
+        fl = prep_value<D, S, ST, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low,
                                                                    lim_high, zdt, SECOND_ORDER, sfix + (s + i), A.N);
       } else {
-        HangStencil<D, double> st;
+        using ST = HangStencil<D, double, WT>;
+        ST st;
         st.load(rec, c.ext_of(A.ext, i), A.geom);
-        fl = prep_value<D, S, HangStencil<D, double>, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low,
+        fl = prep_value<D, S, ST, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low,
                                                                     lim_high, zdt, SECOND_ORDER, sfix + (s + i),
                                                                     A.N);
       }
@@ -693,24 +730,24 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
   }
 }
 
-template <int D, class S, bool SECOND_ORDER>
+template <int D, class S, bool SECOND_ORDER, bool WT = false>
 __global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_per_eu(CASL_TILE_WAVES_F64)))
     k_tile_prep(TileArgs<double> A, const uint8_t *__restrict__ mask,
                                                           double lim_low, double lim_high, double zdt,
                                                           uint16_t *__restrict__ flags, S *__restrict__ sfix) {
   __shared__ double phis[TileLimits<D>::LMAX];
   __shared__ double dds[SECOND_ORDER ? D * TileLimits<D>::DMAX : 1];
-  tile_prep<D, S, SECOND_ORDER, TILE_BLOCK_F64>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds, mask, lim_low,
+  tile_prep<D, S, SECOND_ORDER, TILE_BLOCK_F64, WT>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds, mask, lim_low,
                                             lim_high, zdt, flags, sfix);
 }
 
-template <int D, class R, bool SECOND_ORDER, bool RK_AVG>
+template <int D, class R, bool SECOND_ORDER, bool RK_AVG, bool WT = false>
 __global__ void __launch_bounds__(stage_block<R>())
     __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? CASL_TILE_WAVES_F32 : CASL_TILE_WAVES_F64)))
     k_tile_stage(TileArgs<R> A) {
   __shared__ R phis[TileLimits<D>::LMAX];
   __shared__ R dds[SECOND_ORDER ? D * TileLimits<D>::DMAX : 1];
-  tile_stage<D, R, SECOND_ORDER, RK_AVG, stage_block<R>()>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds);
+  tile_stage<D, R, SECOND_ORDER, RK_AVG, stage_block<R>(), WT>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds);
 }
 
 }  // namespace dev

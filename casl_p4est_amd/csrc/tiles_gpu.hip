@@ -50,6 +50,7 @@ enum : int {
   BAD_UNITS = 32,      // a transverse offset that is not a multiple of the finest cell
   BAD_VERIFY = 64,     // a decoded record differs from the tables
   BAD_BOUNDS = 128,    // the independent bounds check failed
+  ODD_WEIGHT = 256,    // no error: a regular face whose transverse offsets are not base * 2^-l
 };
 
 // The flattened tables on the device (FP64 distances), as casl_flat_stencil.
@@ -452,6 +453,12 @@ __device__ int encode(const DTab<D> &t, const TileView &v, const TileLocal<D> &l
   return k;
 }
 
+// v is 0 or base times a power of two
+__device__ __forceinline__ bool scale_multiple(double b, double v) {
+  int eb = 0, ev = 0;
+  return v == 0.0 || frexp(b, &eb) == frexp(v, &ev);
+}
+
 // The host builder's verify(): the decoded record reproduces the tables
 // (distances bit-exact, one nonzero-weight corner on a face without a
 // hanging arm).  Its slots are what encode() looked up for the same nodes
@@ -481,6 +488,10 @@ __device__ void verify(const DTab<D> &t, const TileView &v, int64_t n, const Til
       int nz = 0;
       for (int c = 0; c < C; ++c) nz += (w[c] != 0.0) ? 1 : 0;
       if (nz != 1) flag(bad, BAD_VERIFY);
+      int t1, t2;
+      transverse(D, f >> 1, t1, t2);
+      for (int k = 0; k < 2 * (D - 1); ++k)
+        if (!scale_multiple(base[k < 2 ? t1 : t2], t.dt(f, k, n))) flag(bad, ODD_WEIGHT);
       continue;
     }
     const uint16_t *fe = e + 1 + q * SW;
@@ -949,7 +960,8 @@ void build(const DTab<D> &tab, casl_stencil *st, hipStream_t s) {
   to32(urs, st->t_urec_start);
   to32(xs, st->t_ext_start);
   b = read_back(bad.p, s);
-  if (b) throw std::runtime_error(bad_reason(b));
+  if (b & ~ODD_WEIGHT) throw std::runtime_error(bad_reason(b));
+  st->regular_weights = (b & ODD_WEIGHT) == 0;
   // geometry and counts
   st->n_tiles = nt;
   st->n_halo = n_halo;
@@ -965,7 +977,7 @@ void build(const DTab<D> &tab, casl_stencil *st, hipStream_t s) {
   hipLaunchKernelGGL(k_validate<D>, dim3(unsigned(nt)), dim3(BLOCK), 0, s, tile_args<float>(st), N, bad.p);
   HIP_CHECK(hipGetLastError());
   b = read_back(bad.p, s);
-  if (b) {
+  if (b & ~ODD_WEIGHT) {
     st->tiled = false;
     throw std::runtime_error(bad_reason(b));
   }
