@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "reinit_device.hpp"
 #include "tiles_device.hpp"
@@ -50,12 +51,14 @@ __global__ void __launch_bounds__(BLOCK) k_advect(TB t, const double *__restrict
 // T u H1, then advect_value for T.  out = result, or (RK_AVG) out = (out +
 // result) / 2.  The loads a node needs (its record, slot and vn, and the
 // value being averaged) are issued before the first barrier.
-template <int D, bool RK_AVG, bool WT>
-__global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_per_eu(CASL_TILE_WAVES_F64)))
+template <int D, bool RK_AVG, bool WT, bool SMALL>
+__global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
+    __attribute__((amdgpu_waves_per_eu((tile_waves<D, double, SMALL>()))))
     k_tile_advect(TileArgs<double> A, const double *__restrict__ vn, double dt) {
-  constexpr int DMAX = TileLimits<D>::DMAX;
-  constexpr int KT = TileLimits<D>::TMAX / TILE_BLOCK_F64;
-  __shared__ double phis[TileLimits<D>::LMAX];
+  using LIM = TileLimits<D, SMALL>;
+  constexpr int DMAX = LIM::DMAX, BT = tile_block<D, double, SMALL>();
+  constexpr int KT = (LIM::TMAX + BT - 1) / BT;
+  __shared__ double phis[LIM::LMAX];
   __shared__ double dds[D * DMAX];
   const int tile = xcd_tile(int(blockIdx.x), int(gridDim.x));
   TileCtx<D> c;
@@ -66,26 +69,26 @@ __global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_pe
   int tslot[KT];
 #pragma unroll
   for (int k = 0; k < KT; ++k) {
-    const int i = int(threadIdx.x) + k * TILE_BLOCK_F64;
+    const int i = int(threadIdx.x) + k * BT;
     if (i < nT) tslot[k] = fetch_record<D>(A, c, i, trec[k]);
   }
-  for (int j = threadIdx.x; j < nT; j += TILE_BLOCK_F64) phis[j] = A.phin[s + j];
-  for (int j = threadIdx.x; j < nH; j += TILE_BLOCK_F64) phis[nT + j] = A.phin[A.halo[hb + j]];
+  for (int j = threadIdx.x; j < nT; j += BT) phis[j] = A.phin[s + j];
+  for (int j = threadIdx.x; j < nH; j += BT) phis[nT + j] = A.phin[A.halo[hb + j]];
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < KT; ++k) {
-    const int i = int(threadIdx.x) + k * TILE_BLOCK_F64;
-    if (i < nT) tile_pass_a<D, double, WT>(A, c, ufast, trec[k], tslot[k], i, phis, dds);
+    const int i = int(threadIdx.x) + k * BT;
+    if (i < nT) tile_pass_a<D, double, WT, SMALL>(A, c, ufast, trec[k], tslot[k], i, phis, dds);
   }
-  for (int i = nT + int(threadIdx.x); i < nT + nH1; i += TILE_BLOCK_F64) {
+  for (int i = nT + int(threadIdx.x); i < nT + nH1; i += BT) {
     RecRegs r;
     const int js = fetch_record<D>(A, c, i, r);
-    tile_pass_a<D, double, WT>(A, c, ufast, r, js, i, phis, dds);
+    tile_pass_a<D, double, WT, SMALL>(A, c, ufast, r, js, i, phis, dds);
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < KT; ++k) {
-    const int i = int(threadIdx.x) + k * TILE_BLOCK_F64;
+    const int i = int(threadIdx.x) + k * BT;
     if (i >= nT) continue;
     int j = tslot[k];
     double r;
@@ -145,24 +148,24 @@ void run_advect(casl_stencil *st, double *phi, const double *vn, const double *v
   if (st->use_tiles(true)) {
     st->phi0.ensure(N);
     TileArgs<double> ta = tile_args<double>(st);
-    const dim3 g(unsigned(st->n_tiles)), b(TILE_BLOCK_F64);
-    const bool wt = st->weighted_tiles();
-    ta.phin = phi;
-    ta.out = st->phi0.p;
-    prof_begin("k_tile_advect", s);
-    if (wt)
-      hipLaunchKernelGGL((k_tile_advect<D, false, true>), g, b, 0, s, ta, vn, dt);
-    else
-      hipLaunchKernelGGL((k_tile_advect<D, false, false>), g, b, 0, s, ta, vn, dt);
-    prof_end("k_tile_advect", s);
-    ta.phin = st->phi0.p;
-    ta.out = phi;
-    prof_begin("k_tile_advect", s);
-    if (wt)
-      hipLaunchKernelGGL((k_tile_advect<D, true, true>), g, b, 0, s, ta, vnp1 ? vnp1 : vn, dt);
-    else
-      hipLaunchKernelGGL((k_tile_advect<D, true, false>), g, b, 0, s, ta, vnp1 ? vnp1 : vn, dt);
-    prof_end("k_tile_advect", s);
+    const dim3 g(unsigned(st->n_tiles));
+    auto stage = [&](auto rk, const double *in, double *out, const double *v) {
+      ta.phin = in;
+      ta.out = out;
+      prof_begin("k_tile_advect", s);
+      auto launch = [&](auto wt, auto small) {
+        constexpr bool SM = decltype(small)::value;
+        hipLaunchKernelGGL((k_tile_advect<D, decltype(rk)::value, decltype(wt)::value, SM>), g,
+                           dim3(tile_block<D, double, SM>()), 0, s, ta, v, dt);
+      };
+      if (st->weighted_tiles())
+        st->small ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{});
+      else
+        st->small ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{});
+      prof_end("k_tile_advect", s);
+    };
+    stage(std::false_type{}, phi, st->phi0.p, vn);
+    stage(std::true_type{}, st->phi0.p, phi, vnp1 ? vnp1 : vn);
     HIP_CHECK(hipGetLastError());
     return;
   }

@@ -368,7 +368,7 @@ void build_batch_tiles(casl_batch *B, const casl_flat_stencil *trees, const std:
   parallel_for(nt, [&](int64_t b, int64_t e) {
     for (int64_t k = b; k < e; ++k) {
       try {
-        build_tiles(trees[k], hosts[size_t(k)]);
+        build_tiles(trees[k], hosts[size_t(k)], false);
         validate_tile_host(hosts[size_t(k)], D, trees[k].n_nodes);
       } catch (const std::exception &ex) {
         errs[size_t(k)] = ex.what();

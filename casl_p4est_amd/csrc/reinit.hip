@@ -321,13 +321,19 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
     // flags and s_fix in tile-record order, the order the tiled stages read them
     TileArgs<double> tp = tile_args<double>(st);
     tp.phin = B.phi0;
-    const dim3 g(unsigned(st->n_tiles)), b(TILE_BLOCK_F64);
+    const dim3 g(unsigned(st->n_tiles));
     prof_begin("k_tile_prep", s);
-    auto prep = [&](auto second, auto wt) {
-      hipLaunchKernelGGL((k_tile_prep<D, R, decltype(second)::value, decltype(wt)::value>), g, b, 0, s, tp, mask,
-                         lim_low, lim_high, st->zdt, B.flags, sfix);
+    auto prep = [&](auto second, auto wt, auto small) {
+      constexpr bool SM = decltype(small)::value;
+      hipLaunchKernelGGL((k_tile_prep<D, R, decltype(second)::value, decltype(wt)::value, SM>), g,
+                         dim3(tile_block<D, double, SM>()), 0, s, tp, mask, lim_low, lim_high, st->zdt, B.flags, sfix);
     };
-    with_weights<R>(wt_tiles, [&](auto wt) { so ? prep(std::true_type{}, wt) : prep(std::false_type{}, wt); });
+    with_weights<R>(wt_tiles, [&](auto wt) {
+      if (st->small)
+        so ? prep(std::true_type{}, wt, std::true_type{}) : prep(std::false_type{}, wt, std::true_type{});
+      else
+        so ? prep(std::true_type{}, wt, std::false_type{}) : prep(std::false_type{}, wt, std::false_type{});
+    });
     prof_end("k_tile_prep", s);
   } else {
     prof_begin("k_prep", s);
@@ -383,11 +389,14 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
   auto tile_stage = [&](const R *in, R *out, bool avg) {
     ta.phin = in;
     ta.out = out;
-    const dim3 g(unsigned(st->n_tiles)), b(stage_block<R>());
+    const dim3 g(unsigned(st->n_tiles));
     prof_begin("k_tile_stage", s);
     auto launch = [&](auto second, auto rk, auto wt) {
-      hipLaunchKernelGGL(
-          (k_tile_stage<D, R, decltype(second)::value, decltype(rk)::value, decltype(wt)::value>), g, b, 0, s, ta);
+      constexpr bool SO = decltype(second)::value, RK = decltype(rk)::value, WT = decltype(wt)::value;
+      if (st->small)
+        hipLaunchKernelGGL((k_small_stage<D, R, SO, RK, WT>), g, dim3(tile_block<D, R, true>()), 0, s, ta);
+      else
+        hipLaunchKernelGGL((k_tile_stage<D, R, SO, RK, WT>), g, dim3(tile_block<D, R, false>()), 0, s, ta);
     };
     with_weights<R>(wt_tiles, [&](auto wt) {
       if (so)
@@ -449,8 +458,7 @@ void validate_tile_host(const TileHost &H, int D, int64_t n_nodes) {
   const int F = 2 * D, C = 1 << (D - 1);
   const int WORDS = D == 2 ? HangExt<2>::WORDS : HangExt<3>::WORDS, SW = D == 2 ? HangExt<2>::SW : HangExt<3>::SW;
   const int UW = D == 2 ? UniRec<2>::WORDS : UniRec<3>::WORDS;
-  const int LMAX = D == 2 ? TileLimits<2>::LMAX : TileLimits<3>::LMAX;
-  const int DMAX = D == 2 ? TileLimits<2>::DMAX : TileLimits<3>::DMAX;
+  const int LMAX = tile_caps(D, H.small).lmax, DMAX = tile_caps(D, H.small).dmax;
   const int64_t nt = int64_t(H.tile_start.size()) - 1;
   if (H.tile_start.front() != 0 || H.tile_start.back() != n_nodes)
     throw std::runtime_error("tile ranges do not cover the nodes");
@@ -556,6 +564,7 @@ void upload_tile_host(const TileHost &H, int64_t n_nodes, casl_stencil *st) {
   st->n_uniform = int64_t(H.urec_start.back());
   st->n_irregular = H.n_irregular;
   st->regular_weights = H.regular_weights;
+  st->small = H.small;
   for (int a = 0; a < 3; ++a) {
     st->geom_base[a] = H.size[a];
     st->geom_unit[a] = H.size[a] * std::ldexp(1.0, -H.lmax);
@@ -569,20 +578,14 @@ void upload_tile_tables(const casl_flat_stencil *tab, casl_stencil *st) {
   st->tiled = false;
   TileHost H;
   try {
-    build_tiles(*tab, H);
+    build_tiles(*tab, H, small_tiles(tab->dim, tab->n_nodes));
   } catch (const std::exception &e) {
     st->tile_error = e.what();
     return;
   }
   validate_tile_host(H, tab->dim, tab->n_nodes);
   upload_tile_host(H, tab->n_nodes, st);
-  // One block per tile: a grid of fewer tiles than compute units leaves most
-  // of the chip idle, and there the grid-wide kernels (more, smaller blocks)
-  // measured faster (the 15-tile 2D star: 9.5e8 against 7.7e8 FP64
-  // node-iterations/s).  casl_stencil_set_path overrides the choice.
-  hipDeviceProp_t prop;
-  HIP_CHECK(hipGetDeviceProperties(&prop, st->device));
-  st->path = st->n_tiles >= int64_t(prop.multiProcessorCount) ? CASL_PATH_TILED : CASL_PATH_TWO_PASS;
+  st->default_path();
 }
 
 void upload_tables(const casl_flat_stencil *tab, casl_stencil *st, bool with_tiles, bool allow_fp64_copy) {
@@ -692,6 +695,14 @@ void prof_end(const char *kernel, hipStream_t s) {
 
 }  // namespace casl
 
+void casl_stencil::default_path() {
+  hipDeviceProp_t prop;
+  HIP_CHECK(hipGetDeviceProperties(&prop, device));
+  compute_units = prop.multiProcessorCount;
+  full_tiles = (N + casl::tile_caps(dim, false).tmax - 1) / casl::tile_caps(dim, false).tmax;
+  path = CASL_PATH_TILED;
+}
+
 extern "C" {
 
 int casl_profile_enable(int enable) {
@@ -740,6 +751,7 @@ int casl_stencil_set_path(casl_stencil_t *st, int path) {
     if (!st) throw std::invalid_argument("null stencil");
     if (path != CASL_PATH_TILED && path != CASL_PATH_TWO_PASS) throw std::invalid_argument("unknown path");
     st->path = path;
+    st->path_chosen = true;
   });
 }
 
@@ -769,7 +781,7 @@ int casl_tile_plan(const casl_flat_stencil *tables, int64_t *n_tiles, int64_t *n
     if (!tables) throw std::invalid_argument("null tables");
     validate_tables(tables);
     TileHost H;
-    build_tiles(*tables, H);
+    build_tiles(*tables, H, small_tiles(tables->dim, tables->n_nodes));
     validate_tile_host(H, tables->dim, tables->n_nodes);
     const int64_t nt = int64_t(H.tile_start.size()) - 1;
     const int W = tables->dim == 2 ? HangExt<2>::WORDS : HangExt<3>::WORDS;
@@ -794,7 +806,7 @@ int casl_stencil_tile_check(const casl_stencil_t *st, const casl_flat_stencil *t
     *equal = 0;
     TileHost H;
     try {
-      build_tiles(*tables, H);
+      build_tiles(*tables, H, small_tiles(tables->dim, tables->n_nodes));
     } catch (const std::exception &e) {
       // neither encoding exists: equal
       if (!st->tiled) *equal = 1;

@@ -450,7 +450,9 @@ struct casl_stencil {
   casl::DevBuf<unsigned long long> red;
   // tiled encoding (tiles.hpp)
   bool tiled = false;
+  bool small = false;      // the tiles are small ones (TileLimits<D, true>)
   int path = CASL_PATH_TILED;
+  bool path_chosen = false;  // by casl_stencil_set_path
   int64_t n_tiles = 0, n_halo = 0, n_records = 0, n_irregular = 0, n_uniform = 0;
   double geom_base[3] = {0, 0, 0}, geom_unit[3] = {0, 0, 0};
   std::string tile_error;
@@ -534,9 +536,24 @@ struct casl_stencil {
   // origin that rounds the transverse offsets).  20 RK2 iterations on the
   // 2.0M-node octree of 64 spheres in [0, 3]^3: 19.6 ms on the grid-wide
   // kernels, 3.03 ms on these.
+  //
+  // Mixed calls on a grid of fewer than one full-size tile per compute unit
+  // whose cells are not powers of two stay on the grid-wide kernels unless
+  // the caller picks the tiles: FP32 rounds the weighted form there, the
+  // tiles take the corner's value, and a default call keeps its results.
   bool use_tiles(bool fp64) const {
-    return tiled && path == CASL_PATH_TILED && (!fp64 || dyadic_geometry() || regular_weights);
+    if (!tiled || path != CASL_PATH_TILED) return false;
+    if (dyadic_geometry()) return true;
+    return fp64 ? regular_weights : (path_chosen || full_tiles >= compute_units);
   }
+  int64_t full_tiles = 0;  // N over the full-size tile, rounded up
+  int compute_units = 0;
+  // Tiles wherever there is an encoding: one fused kernel per stage against
+  // pass A and pass B.  Per RK2 stage (us, FP64 / mixed, two-pass and tiled):
+  // 2D 727 nodes 7.4 / 7.4 and 7.0 / 5.4, 14.7K 7.8 / 7.8 and 7.1 / 5.8, 119K
+  // 10.2 / 8.0 and 7.8 / 6.3; 3D 11.8K 16.2 / 10.1 and 12.1 / 8.4, 51K 19.7 /
+  // 11.0 and 11.3 / 8.1, 301K 69.7 / 40.1 and 18.7 / 13.0.
+  void default_path();
   bool weighted_tiles() const { return !dyadic_geometry(); }
 };
 

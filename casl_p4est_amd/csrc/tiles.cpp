@@ -25,7 +25,9 @@ struct Builder {
   double unit[3] = {0, 0, 0};
   mutable std::atomic<bool> regular_weights{true};
 
-  explicit Builder(const casl_flat_stencil &t) : tab(t), N(t.n_nodes) {}
+  const TileCaps caps;
+
+  Builder(const casl_flat_stencil &t, bool small) : tab(t), N(t.n_nodes), caps(tile_caps(D, small)) {}
 
   int32_t nbr(int f, int c, int64_t n) const { return tab.nbr[(int64_t(f) * C + c) * N + n]; }
   double d(int f, int64_t n) const { return tab.d[int64_t(f) * N + n]; }
@@ -164,7 +166,7 @@ struct Builder {
     }
     std::sort(t.h1.begin(), t.h1.end());
     t.h1.erase(std::unique(t.h1.begin(), t.h1.end()), t.h1.end());
-    if (nT + int64_t(t.h1.size()) > TileLimits<D>::DMAX) return false;
+    if (nT + int64_t(t.h1.size()) > caps.dmax) return false;
     for (int32_t h : t.h1) {
       const int k = needed(h, buf.data());
       for (int i = 0; i < k; ++i) {
@@ -176,7 +178,7 @@ struct Builder {
     }
     std::sort(t.h2.begin(), t.h2.end());
     t.h2.erase(std::unique(t.h2.begin(), t.h2.end()), t.h2.end());
-    return nT + int64_t(t.h1.size()) + int64_t(t.h2.size()) <= TileLimits<D>::LMAX;
+    return nT + int64_t(t.h1.size()) + int64_t(t.h2.size()) <= caps.lmax;
   }
 
   // The record of node n; for a node with hanging faces also its extension
@@ -361,7 +363,7 @@ struct Builder {
     scan_scales();
     if (!tile_scales_supported(base, D))
       throw std::runtime_error("cells that are not cubes on a box whose edges are not dyadic");
-    const int64_t nCand = (N + TileLimits<D>::TMAX - 1) / TileLimits<D>::TMAX;
+    const int64_t nCand = (N + caps.tmax - 1) / caps.tmax;
     std::vector<std::vector<Tile>> parts(nCand);
     std::atomic<int64_t> cursor{0};
     std::string err;
@@ -373,8 +375,8 @@ struct Builder {
           const int64_t i = cursor.fetch_add(1);
           if (i >= nCand) break;
           try {
-            const int32_t s = int32_t(i * TileLimits<D>::TMAX);
-            const int32_t e = int32_t(std::min<int64_t>(N, (i + 1) * TileLimits<D>::TMAX));
+            const int32_t s = int32_t(i * caps.tmax);
+            const int32_t e = int32_t(std::min<int64_t>(N, (i + 1) * caps.tmax));
             cut(s, e, parts[i]);
           } catch (const std::exception &x) {
             std::lock_guard<std::mutex> g(emu);
@@ -431,12 +433,13 @@ struct Builder {
 
 }  // namespace
 
-void build_tiles(const casl_flat_stencil &tab, TileHost &out) {
+void build_tiles(const casl_flat_stencil &tab, TileHost &out, bool small) {
+  out.small = small;
   if (tab.dim == 2) {
-    Builder<2> b(tab);
+    Builder<2> b(tab, small);
     b.run(out);
   } else {
-    Builder<3> b(tab);
+    Builder<3> b(tab, small);
     b.run(out);
   }
 }

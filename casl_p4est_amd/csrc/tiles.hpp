@@ -154,16 +154,45 @@ constexpr uint16_t HANG_NONE = 15;
 #ifndef CASL_TILE_T3
 #define CASL_TILE_T3 2048
 #endif
-template <int D>
+//
+// SMALL: the tiles of a grid too small to give every compute unit a full-size
+// tile.  There a stage is the latency of one tile, not bandwidth: tiles of 256
+// nodes spread the grid over the chip, and DMAX is also the block size of
+// their kernels, so every node of T u H1 has a thread of its own.
+template <int D, bool SMALL = false>
 struct TileLimits;
 template <>
-struct TileLimits<2> {
+struct TileLimits<2, false> {
   static constexpr int TMAX = CASL_TILE_T2, LMAX = 2 * CASL_TILE_T2, DMAX = 3 * CASL_TILE_T2 / 2;
 };
 template <>
-struct TileLimits<3> {
+struct TileLimits<3, false> {
   static constexpr int TMAX = CASL_TILE_T3, LMAX = 4 * CASL_TILE_T3, DMAX = 2 * CASL_TILE_T3;
 };
+template <>
+struct TileLimits<2, true> {
+  static constexpr int TMAX = 256, LMAX = 768, DMAX = 512;
+};
+template <>
+struct TileLimits<3, true> {
+  static constexpr int TMAX = 256, LMAX = 1536, DMAX = 768;
+};
+// The same at run time.
+struct TileCaps {
+  int tmax, lmax, dmax;
+};
+inline TileCaps tile_caps(int dim, bool small) {
+  if (dim == 2)
+    return small ? TileCaps{TileLimits<2, true>::TMAX, TileLimits<2, true>::LMAX, TileLimits<2, true>::DMAX}
+                 : TileCaps{TileLimits<2>::TMAX, TileLimits<2>::LMAX, TileLimits<2>::DMAX};
+  return small ? TileCaps{TileLimits<3, true>::TMAX, TileLimits<3, true>::LMAX, TileLimits<3, true>::DMAX}
+               : TileCaps{TileLimits<3>::TMAX, TileLimits<3>::LMAX, TileLimits<3>::DMAX};
+}
+// Grids up to this many nodes take small tiles.  Per RK2 stage (us, FP64 /
+// mixed) on small and full-size tiles: 2D 119K nodes 7.8 / 6.3 and 10.5 / 7.9,
+// 237K 11.6 / 7.6 and 10.4 / 8.0; 3D 119K 15.6 / 9.5 and 18.5 / 12.6, 180K
+// 20.4 / 13.6 and 19.1 / 12.9.
+inline bool small_tiles(int dim, int64_t n_nodes) { return n_nodes <= (dim == 2 ? 3 << 16 : 5 << 15); }
 // the uniform record's fields hold every LDS index and slot of a tile
 static_assert(TileLimits<2>::LMAX <= (1 << UniRec<2>::IDX_BITS) && TileLimits<2>::DMAX <= (1 << UniRec<2>::SLOT_BITS),
               "2D tile limits exceed the uniform record's fields");
@@ -189,6 +218,7 @@ inline bool tile_scales_supported(const double *base, int dim) {
 
 struct TileHost {
   int dim = 0;
+  bool small = false;       // cut by TileLimits<dim, true>
   int lmax = 0;             // finest arm level present
   double size[3] = {1, 1, 1};  // tree size per axis (box edge)
   std::vector<int32_t> tile_start;  // [ntiles + 1] node ranges
@@ -211,7 +241,8 @@ struct TileHost {
 
 // Builds the tiled encoding of a flattened stencil; throws std::runtime_error
 // when the stencil cannot be encoded exactly (then the grid-wide kernels are
-// used instead).  box sizes are recovered from the arm lengths.
-void build_tiles(const casl_flat_stencil &tab, TileHost &out);
+// used instead).  box sizes are recovered from the arm lengths.  small: cut
+// by the limits of small tiles.
+void build_tiles(const casl_flat_stencil &tab, TileHost &out, bool small);
 
 }  // namespace casl

@@ -194,6 +194,22 @@ __device__ __forceinline__ TileRec uni_as_rec(const uint32_t *w, int &slot) {
   return r;
 }
 
+// An extension record in registers.
+template <int D>
+struct ExtRegs {
+  static constexpr int NW = HangExt<D>::WORDS / 2;  // 32-bit words (the record is whole 8-byte words)
+  uint32_t e[NW];
+  __device__ __forceinline__ void load(const uint16_t *__restrict__ xrec) {
+    const uint2 *src = reinterpret_cast<const uint2 *>(xrec);
+#pragma unroll
+    for (int i = 0; i < NW / 2; ++i) {
+      const uint2 v = src[i];
+      e[2 * i] = v.x;
+      e[2 * i + 1] = v.y;
+    }
+  }
+};
+
 // Stencil of a node with hanging arms: the record's one corner per face, and
 // for the faces that hang (at most D - 1) the extension record's corners and
 // transverse offsets.  idx / dt serve any face (the per-face functions); the
@@ -204,9 +220,8 @@ struct HangStencil : DecodedDist<D, R, WT> {
   static constexpr bool SLOTS = true;
   static constexpr int F = 2 * D, C = 1 << (D - 1);
   static constexpr int NH = HangExt<D>::NH, WORDS = HangExt<D>::WORDS, SW = HangExt<D>::SW;
-  static constexpr int NW = WORDS / 2;  // 32-bit words (the record is whole 8-byte words)
   uint16_t id[F];
-  uint32_t e[NW];
+  ExtRegs<D> ex;
   bool pow2;
   uint32_t geo;
   R base[D], inv_base[D];  // the geometry's (uniform values)
@@ -261,7 +276,7 @@ struct HangStencil : DecodedDist<D, R, WT> {
     r.ut2 = ldexp(ua, d2);
     return r;
   }
-  __device__ __forceinline__ uint32_t word(int i) const { return (e[i >> 1] >> (16 * (i & 1))) & 0xffffu; }
+  __device__ __forceinline__ uint32_t word(int i) const { return (ex.e[i >> 1] >> (16 * (i & 1))) & 0xffffu; }
   // face of hanging slot q (HANG_NONE when the node has fewer)
   __device__ __forceinline__ int hface(int q) const {
     return D == 2 ? int(word(0)) : int((word(0) >> (4 * q)) & 15u);
@@ -299,15 +314,14 @@ struct HangStencil : DecodedDist<D, R, WT> {
   }
   // rec: the node's record; xrec: its extension record (WORDS uint16)
   __device__ __forceinline__ void load(const TileRec &rec, const uint16_t *__restrict__ xrec, const TileGeom<R> &g) {
+    ExtRegs<D> x;
+    x.load(xrec);
+    load(rec, x, g);
+  }
+  __device__ __forceinline__ void load(const TileRec &rec, const ExtRegs<D> &x, const TileGeom<R> &g) {
 #pragma unroll
     for (int f = 0; f < F; ++f) id[f] = rec.idx[f];
-    const uint2 *src = reinterpret_cast<const uint2 *>(xrec);
-#pragma unroll
-    for (int i = 0; i < NW / 2; ++i) {
-      const uint2 v = src[i];
-      e[2 * i] = v.x;
-      e[2 * i + 1] = v.y;
-    }
+    ex = x;
     pow2 = !WT && g.pow2 != 0;
     geo = rec.geo;
 #pragma unroll
@@ -396,6 +410,10 @@ struct TileCtx {
   }
   // other position i: its rank among the tile's non-uniform records
   __device__ __forceinline__ int npos(int i) const { return i < nT ? i - nTu : (nT - nTu) + (i - nT - nH1u); }
+  // position i holds a record with hanging faces
+  __device__ __forceinline__ bool irregular(int i) const {
+    return i < nT ? i >= nTu + int(nreg & 0xffffu) : (i - nT) >= nH1u + int(nreg >> 16);
+  }
   __device__ __forceinline__ const uint16_t *ext_of(const uint16_t *__restrict__ ext, int i) const {
     return hang_record(ext, ext0, nreg, nT - nTu, npos(i), HangExt<D>::WORDS);
   }
@@ -450,11 +468,13 @@ __device__ __forceinline__ int slot_at(const TileCtx<D> &c, int i, const RecRegs
 // Pass A (laplace) of the record at position i into dds[a * DMAX + slot].
 // Uniform records where UniStencil holds (ufast: see TileGeom::uni_fast) take
 // it, the others the general decoding.
-template <int D, class R, bool WT = false>
+// xrec: the extension record of an irregular position, if the caller already
+// has it in registers.
+template <int D, class R, bool WT = false, bool SMALL = false>
 __device__ __forceinline__ void tile_pass_a(const TileArgs<R> &A, const TileCtx<D> &c, bool ufast, const RecRegs &r,
                                             int fetched_slot, int i, const R *__restrict__ phis,
-                                            R *__restrict__ dds) {
-  constexpr int DMAX = TileLimits<D>::DMAX;
+                                            R *__restrict__ dds, const ExtRegs<D> *xrec = nullptr) {
+  constexpr int DMAX = TileLimits<D, SMALL>::DMAX;
   R f000, fnb[2 * D], dd[D];
   int j = fetched_slot;
   if (ufast && c.uniform(i)) {
@@ -469,7 +489,10 @@ __device__ __forceinline__ void tile_pass_a(const TileArgs<R> &A, const TileCtx<
       laplace<D, R>(st, j, phis, f000, fnb, dd);
     } else {
       HangStencil<D, R, WT> st;
-      st.load(rec, c.ext_of(A.ext, i), A.geom);
+      if (xrec)
+        st.load(rec, *xrec, A.geom);
+      else
+        st.load(rec, c.ext_of(A.ext, i), A.geom);
       laplace<D, R>(st, j, phis, f000, fnb, dd);
     }
   }
@@ -491,9 +514,12 @@ __device__ __forceinline__ void tile_pass_a(const TileArgs<R> &A, const TileCtx<
 #endif
 constexpr int TILE_BLOCK = CASL_TILE_BLOCK;
 constexpr int TILE_BLOCK_F64 = CASL_TILE_BLOCK_F64;
-template <class R>
-constexpr int stage_block() {
-  return sizeof(R) == 8 ? TILE_BLOCK_F64 : TILE_BLOCK;
+// Small tiles: one thread per node of T u H1.  A 3D block is 12 waves, three
+// per SIMD in FP64 (up to 168 VGPRs), six in FP32 (80: two blocks per compute
+// unit); a 2D block is 8 waves, four per SIMD over two blocks.
+template <int D, class R, bool SMALL>
+constexpr int tile_block() {
+  return SMALL ? TileLimits<D, true>::DMAX : (sizeof(R) == 8 ? TILE_BLOCK_F64 : TILE_BLOCK);
 }
 
 // One pseudo-time stage of a tile: phi of T u H1 u H2 into LDS, pass A for
@@ -512,6 +538,11 @@ constexpr int stage_block() {
 #ifndef CASL_TILE_WAVES_F64
 #define CASL_TILE_WAVES_F64 4
 #endif
+template <int D, class R, bool SMALL>
+constexpr int tile_waves() {
+  if (SMALL) return D == 2 ? 4 : (sizeof(R) == 8 ? 3 : 6);
+  return sizeof(R) == 8 ? CASL_TILE_WAVES_F64 : CASL_TILE_WAVES_F32;
+}
 // The stage body for one tile, run by a block of BLOCK threads with LDS
 // arrays phis[LMAX] and dds[D * DMAX].  It reads and writes global memory and
 // the LDS arrays only; a caller running several tiles in a row separates them
@@ -676,12 +707,12 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
 // pass A of phi_0 for T u H1 (second order), then flags and s_fix of the
 // tile's nodes, written in record order (tile start + record position), the
 // order the stage body reads them in.  A.phin is phi_0.
-template <int D, class S, bool SECOND_ORDER, int BLOCK, bool WT = false>
+template <int D, class S, bool SECOND_ORDER, int BLOCK, bool WT = false, bool SMALL = false>
 __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, double *__restrict__ phis,
                                           double *__restrict__ dds, const uint8_t *__restrict__ mask,
                                           double lim_low, double lim_high, double zdt,
                                           uint16_t *__restrict__ flags, S *__restrict__ sfix) {
-  constexpr int DMAX = TileLimits<D>::DMAX;
+  constexpr int DMAX = TileLimits<D, SMALL>::DMAX;
   TileCtx<D> c;
   c.load(A, tile);
   const int s = c.s, nT = c.nT, hb = c.hb, nH = c.nH, nH1 = c.nH1;
@@ -693,7 +724,7 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
     for (int i = int(threadIdx.x); i < nT + nH1; i += BLOCK) {
       RecRegs r;
       const int js = fetch_record<D>(A, c, i, r);
-      tile_pass_a<D, double, WT>(A, c, ufast, r, js, i, phis, dds);
+      tile_pass_a<D, double, WT, SMALL>(A, c, ufast, r, js, i, phis, dds);
     }
     __syncthreads();
   }
@@ -730,24 +761,109 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
   }
 }
 
-template <int D, class S, bool SECOND_ORDER, bool WT = false>
-__global__ void __launch_bounds__(TILE_BLOCK_F64) __attribute__((amdgpu_waves_per_eu(CASL_TILE_WAVES_F64)))
-    k_tile_prep(TileArgs<double> A, const uint8_t *__restrict__ mask,
-                                                          double lim_low, double lim_high, double zdt,
-                                                          uint16_t *__restrict__ flags, S *__restrict__ sfix) {
-  __shared__ double phis[TileLimits<D>::LMAX];
-  __shared__ double dds[SECOND_ORDER ? D * TileLimits<D>::DMAX : 1];
-  tile_prep<D, S, SECOND_ORDER, TILE_BLOCK_F64, WT>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds, mask, lim_low,
-                                            lim_high, zdt, flags, sfix);
+template <int D, class S, bool SECOND_ORDER, bool WT = false, bool SMALL = false>
+__global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
+    __attribute__((amdgpu_waves_per_eu((tile_waves<D, double, SMALL>()))))
+    k_tile_prep(TileArgs<double> A, const uint8_t *__restrict__ mask, double lim_low, double lim_high, double zdt,
+                uint16_t *__restrict__ flags, S *__restrict__ sfix) {
+  using LIM = TileLimits<D, SMALL>;
+  __shared__ double phis[LIM::LMAX];
+  __shared__ double dds[SECOND_ORDER ? D * LIM::DMAX : 1];
+  tile_prep<D, S, SECOND_ORDER, tile_block<D, double, SMALL>(), WT, SMALL>(
+      A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds, mask, lim_low, lim_high, zdt, flags, sfix);
 }
 
 template <int D, class R, bool SECOND_ORDER, bool RK_AVG, bool WT = false>
-__global__ void __launch_bounds__(stage_block<R>())
-    __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? CASL_TILE_WAVES_F32 : CASL_TILE_WAVES_F64)))
+__global__ void __launch_bounds__((tile_block<D, R, false>()))
+    __attribute__((amdgpu_waves_per_eu((tile_waves<D, R, false>()))))
     k_tile_stage(TileArgs<R> A) {
   __shared__ R phis[TileLimits<D>::LMAX];
   __shared__ R dds[SECOND_ORDER ? D * TileLimits<D>::DMAX : 1];
-  tile_stage<D, R, SECOND_ORDER, RK_AVG, stage_block<R>(), WT>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds);
+  tile_stage<D, R, SECOND_ORDER, RK_AVG, tile_block<D, R, false>(), WT>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)),
+                                                                       phis, dds);
+}
+
+// One pseudo-time stage of one small tile, one thread per node of T u H1 (the
+// body of tile_stage with every load of a thread's one record issued before
+// the first barrier).  A grid this small is bound by the chain of dependent
+// loads in a stage and by the launch, not by bandwidth, so everything that
+// can be fetched early is: a record's extension is addressed from its
+// position, the subcell distances from the flags, and only the tile's ranges,
+// the halo ids and the phi they name depend on one another.  20 RK2
+// iterations on 14.7K 2D nodes in FP64: 335 us as pass A and pass B kernels,
+// 295 us; 119K 2D nodes mixed, from a graph: 323 and 254 us.
+template <int D, class R, bool SECOND_ORDER, bool RK_AVG, bool WT>
+__global__ void __launch_bounds__((tile_block<D, R, true>()))
+    __attribute__((amdgpu_waves_per_eu((tile_waves<D, R, true>()))))
+    k_small_stage(TileArgs<R> A) {
+  using LIM = TileLimits<D, true>;
+  constexpr int DMAX = LIM::DMAX, BLOCK = tile_block<D, R, true>(), F = 2 * D;
+  static_assert(LIM::TMAX <= BLOCK && DMAX <= BLOCK, "one thread per node of T u H1");
+  __shared__ R phis[LIM::LMAX];
+  __shared__ R dds[SECOND_ORDER ? D * DMAX : 1];
+  TileCtx<D> c;
+  c.load(A, xcd_tile(int(blockIdx.x), int(gridDim.x)));
+  const bool ufast = A.geom.template uni_fast<WT>();
+  const int i = int(threadIdx.x), s = c.s;
+  const bool own = i < c.nT, active = i < c.nT + (SECOND_ORDER ? c.nH1 : 0);
+  constexpr int KH = (LIM::LMAX + BLOCK - 1) / BLOCK;
+  int hid[KH];
+#pragma unroll
+  for (int k = 0; k < KH; ++k)
+    if (i + k * BLOCK < c.nH) hid[k] = A.halo[c.hb + i + k * BLOCK];
+  RecRegs rec{};
+  ExtRegs<D> ext{};
+  int js = 0;
+  uint16_t fl = 0;
+  if (active) {
+    js = fetch_record<D>(A, c, i, rec);
+    if (c.irregular(i)) ext.load(c.ext_of(A.ext, i));
+  }
+  if (own) fl = A.flags[s + i];
+  R tv = R(0), hv[KH], prev = R(0), sf[F];
+  if (own) tv = A.phin[s + i];
+#pragma unroll
+  for (int k = 0; k < KH; ++k)
+    if (i + k * BLOCK < c.nH) hv[k] = A.phin[hid[k]];
+  const unsigned cross = (fl >> 3) & ((1u << F) - 1);
+#pragma unroll
+  for (int f = 0; f < F; ++f) sf[f] = (cross & (1u << f)) ? A.sfix[int64_t(f) * A.N + s + i] : R(0);
+  if constexpr (RK_AVG) {
+    if (own) prev = A.out[s + slot_at<D>(c, i, rec, js)];
+  }
+  if (own) phis[i] = tv;
+#pragma unroll
+  for (int k = 0; k < KH; ++k)
+    if (i + k * BLOCK < c.nH) phis[c.nT + i + k * BLOCK] = hv[k];
+  __syncthreads();
+  if constexpr (SECOND_ORDER) {
+    if (active) tile_pass_a<D, R, WT, true>(A, c, ufast, rec, js, i, phis, dds, &ext);
+    __syncthreads();
+  }
+  if (!own) return;
+  int j = js;
+  R r;
+  if (ufast && i < c.nTu) {
+    using ST = UniStencil<D, R, WT>;
+    ST st;
+    j = st.load(rec.w, A.geom);
+    r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, 0, sf, 1, A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
+  } else {
+    const TileRec tr = record_at<D>(c, i, rec, j);
+    const uint8_t w = uint8_t((tr.geo >> 24) & 63u);
+    if (!(tr.geo & GEO_IRREGULAR)) {
+      using ST = RegStencil<D, R, WT>;
+      ST st;
+      st.load(tr, A.geom);
+      r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, sf, 1, A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
+    } else {
+      using ST = HangStencil<D, R, WT>;
+      ST st;
+      st.load(tr, ext, A.geom);
+      r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, sf, 1, A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
+    }
+  }
+  A.out[s + j] = RK_AVG ? R(0.5) * (prev + r) : r;
 }
 
 }  // namespace dev

@@ -290,13 +290,12 @@ __global__ void k_h2(DTab<D> t, const int32_t *__restrict__ ts, const uint64_t *
 }
 
 // 1 where a tile exceeds its LDS limits (the host's halo() test)
-template <int D>
 __global__ void k_tile_fits(const int32_t *__restrict__ ts, int nt, const int64_t *__restrict__ h1seg,
-                            const int64_t *__restrict__ h2seg, uint8_t *__restrict__ fail) {
+                            const int64_t *__restrict__ h2seg, TileCaps caps, uint8_t *__restrict__ fail) {
   const int t = int(blockIdx.x) * blockDim.x + int(threadIdx.x);
   if (t >= nt) return;
   const int64_t nT = ts[t + 1] - ts[t], n1 = h1seg[t + 1] - h1seg[t], n2 = h2seg[t + 1] - h2seg[t];
-  fail[t] = (nT + n1 > TileLimits<D>::DMAX || nT + n1 + n2 > TileLimits<D>::LMAX) ? 1 : 0;
+  fail[t] = (nT + n1 > caps.dmax || nT + n1 + n2 > caps.lmax) ? 1 : 0;
 }
 
 // ---------------------------------------------------------------- records
@@ -652,8 +651,9 @@ __global__ void k_emit_halo(const uint64_t *__restrict__ h, int64_t nh, const in
 
 // The independent bounds check of validate_tile_host, one block per tile.
 template <int D>
-__global__ void k_validate(TileArgs<float> A, int64_t N, int *__restrict__ bad) {
-  constexpr int F = 2 * D, C = 1 << (D - 1), LMAX = TileLimits<D>::LMAX, DMAX = TileLimits<D>::DMAX;
+__global__ void k_validate(TileArgs<float> A, int64_t N, TileCaps caps, int *__restrict__ bad) {
+  constexpr int F = 2 * D, C = 1 << (D - 1), DMAX = TileLimits<D>::DMAX;
+  static_assert(TileLimits<D, true>::DMAX <= DMAX, "the bit set covers the larger tiles");
   constexpr int WORDS = HangExt<D>::WORDS, SW = HangExt<D>::SW;
   __shared__ uint32_t seen[(DMAX + 31) / 32];
   const int tile = int(blockIdx.x);
@@ -664,7 +664,7 @@ __global__ void k_validate(TileArgs<float> A, int64_t N, int *__restrict__ bad) 
   const int nTn = c.nT - c.nTu, nH1n = c.nH1 - c.nH1u;
   const int nTreg = int(c.nreg & 0xffffu), nH1reg = int(c.nreg >> 16);
   const int nR = A.rec_start[tile + 1] - c.rb, nU = A.urec_start[tile + 1] - c.ub;
-  if (c.nT <= 0 || c.nH1 < 0 || c.nH1 > c.nH || c.nT + c.nH > LMAX || c.nT + c.nH1 > DMAX ||
+  if (c.nT <= 0 || c.nH1 < 0 || c.nH1 > c.nH || c.nT + c.nH > caps.lmax || c.nT + c.nH1 > caps.dmax ||
       nR + nU != c.nT + c.nH1 || c.nTu > c.nT || c.nH1u > c.nH1 || c.nTu + c.nH1u != nU || nTreg > nTn ||
       nH1reg > nH1n || A.ext_start[tile + 1] - c.ext0 != (nTn - nTreg) + (nH1n - nH1reg)) {
     if (threadIdx.x == 0) flag(bad, BAD_BOUNDS);
@@ -807,10 +807,11 @@ void build(const DTab<D> &tab, casl_stencil *st, hipStream_t s) {
   int b = read_back(bad.p, s);
   if (b) throw std::runtime_error(bad_reason(b));
 
-  // tiles: candidates of TMAX nodes, halved where the halo does not fit
-  constexpr int TMAX = TileLimits<D>::TMAX;
+  // tiles: candidates of the tile size, halved where the halo does not fit
+  const bool small = small_tiles(D, N);
+  const TileCaps caps = tile_caps(D, small);
   std::vector<int32_t> starts;
-  for (int64_t x = 0; x < N; x += TMAX) starts.push_back(int32_t(x));
+  for (int64_t x = 0; x < N; x += caps.tmax) starts.push_back(int32_t(x));
   starts.push_back(int32_t(N));
   DevBuf<int32_t> ts;
   DevBuf<uint64_t> keys, h1, h2;
@@ -858,7 +859,7 @@ void build(const DTab<D> &tab, casl_stencil *st, hipStream_t s) {
     // which tiles do not fit
     DevBuf<uint8_t> fail;
     fail.ensure(size_t(nt));
-    hipLaunchKernelGGL(k_tile_fits<D>, dim3(grid_for(nt)), dim3(BLOCK), 0, s, ts.p, nt, h1seg.p, h2seg.p, fail.p);
+    hipLaunchKernelGGL(k_tile_fits, dim3(grid_for(nt)), dim3(BLOCK), 0, s, ts.p, nt, h1seg.p, h2seg.p, caps, fail.p);
     HIP_CHECK(hipGetLastError());
     std::vector<uint8_t> hf(static_cast<size_t>(nt));
     HIP_CHECK(hipMemcpyAsync(hf.data(), fail.p, size_t(nt), hipMemcpyDeviceToHost, s));
@@ -968,13 +969,15 @@ void build(const DTab<D> &tab, casl_stencil *st, hipStream_t s) {
   st->n_records = R;
   st->n_uniform = n_uni;
   st->n_irregular = n_ext;
+  st->small = small;
   for (int a = 0; a < 3; ++a) {
     st->geom_base[a] = sc.base[a];
     st->geom_unit[a] = sc.unit[a];
   }
   st->tiled = true;
   // the independent bounds check before any kernel reads the encoding
-  hipLaunchKernelGGL(k_validate<D>, dim3(unsigned(nt)), dim3(BLOCK), 0, s, tile_args<float>(st), N, bad.p);
+  hipLaunchKernelGGL(k_validate<D>, dim3(unsigned(nt)), dim3(BLOCK), 0, s, tile_args<float>(st), N, caps,
+                     bad.p);
   HIP_CHECK(hipGetLastError());
   b = read_back(bad.p, s);
   if (b & ~ODD_WEIGHT) {
@@ -1036,9 +1039,7 @@ void build_tiles_device(const casl_flat_stencil &dtab, casl_stencil *st, hipStre
     st->tile_error = e.what();
     return;
   }
-  hipDeviceProp_t prop;
-  HIP_CHECK(hipGetDeviceProperties(&prop, st->device));
-  st->path = st->n_tiles >= int64_t(prop.multiProcessorCount) ? CASL_PATH_TILED : CASL_PATH_TWO_PASS;
+  st->default_path();
 }
 
 }  // namespace casl

@@ -72,8 +72,8 @@ class DeviceStencil:
 
     def set_path(self, path):
         """"tiled" (fused stage kernel over LDS-staged Morton tiles; the default
-        when the stencil makes at least one tile per compute unit) or
-        "two_pass" (grid-wide pass A + pass B; the default for smaller grids)."""
+        when the stencil could be tiled) or "two_pass" (grid-wide pass A +
+        pass B)."""
         code = {"tiled": L.CASL_PATH_TILED, "two_pass": L.CASL_PATH_TWO_PASS}[path]
         L.call("casl_stencil_set_path", self._h, code)
 

@@ -96,13 +96,15 @@ int casl_stencil_destroy(casl_stencil_t *st);
 int casl_stencil_info(const casl_stencil_t *st, int32_t *dim, int64_t *n_nodes);
 
 /* Stage kernel selection.  CASL_PATH_TILED: one fused kernel per
- * pseudo-time stage over Morton tiles with LDS-staged halos (the default when
- * the stencil could be tiled into at least one tile per compute unit);
- * CASL_PATH_TWO_PASS: grid-wide pass A + pass B kernels (the default for
- * smaller grids).  A stencil without a tiled encoding (cells that are not
- * cubes, or tile limits exceeded; casl_stencil_tile_info gives the reason)
- * runs CASL_PATH_TWO_PASS whatever was set; get_path returns the path that
- * runs. */
+ * pseudo-time stage over Morton tiles with LDS-staged halos (the default);
+ * CASL_PATH_TWO_PASS: grid-wide pass A + pass B kernels.  A stencil without a
+ * tiled encoding (cells that are not cubes, or tile limits exceeded;
+ * casl_stencil_tile_info gives the reason) runs CASL_PATH_TWO_PASS whatever
+ * was set; get_path returns the path that runs.  Two kinds of call run the
+ * grid-wide kernels on a tiled stencil: FP64 where the tiles could not give
+ * the grid-wide kernels' bits (an origin that rounds the cells' offsets), and
+ * mixed calls, unless set_path chose the tiles, on fewer nodes than one
+ * full-size tile per compute unit whose cell edges are not powers of two. */
 #define CASL_PATH_TILED    0
 #define CASL_PATH_TWO_PASS 1
 int casl_stencil_set_path(casl_stencil_t *st, int path);
