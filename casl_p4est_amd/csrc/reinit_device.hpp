@@ -448,6 +448,11 @@ struct casl_stencil {
   casl::DevBuf<float> phif, tmpf, ddnf, sfixf;
   casl::DevBuf<uint16_t> flags;
   casl::DevBuf<unsigned long long> red;
+  // casl_curvature_grid_samples: arms by face, node states, counts per block
+  casl::DevBuf<int32_t> arms;
+  casl::DevBuf<uint8_t> sample_state;
+  casl::DevBuf<uint32_t> sample_counts;
+  casl::DevBuf<int64_t> sample_first;
   // tiled encoding (tiles.hpp)
   bool tiled = false;
   bool small = false;      // the tiles are small ones (TileLimits<D, true>)

@@ -454,9 +454,8 @@ def grid_samples(ds, phi, h, band, normals=None, kappa=None):
         if cnt.value <= cap:
             break
         cap = cnt.value
-    n = cnt.value
-    order = torch.argsort(node[:n])
-    return feat[:n][order], off[:n][order], node[:n][order], skipped.value
+    n = cnt.value  # the samples come in node order
+    return feat[:n], off[:n], node[:n], skipped.value
 
 
 class UniformBox:
