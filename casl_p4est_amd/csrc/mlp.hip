@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "curv_device.hpp"
+#include "mlp_chain.hpp"
 #include "reinit_device.hpp"
 
 using namespace casl;
@@ -298,11 +299,23 @@ __global__ void __launch_bounds__(256) k_colsum_fin(const float *__restrict__ pa
   if (t == 0) out[c] = red[0];
 }
 
-// Adam on FP32 masters, refreshes the BF16 copy (may be null for biases)
-__global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m, float *__restrict__ v,
-                       uint16_t *__restrict__ p16, int n, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// Adam on FP32 masters, weights then biases in one launch; refreshes the BF16
+// copy of the weights and its transposed copy (in: the input width, 0: none)
+struct AdamVec {
+  float *p;
+  const float *g;
+  float *m, *v;
+};
+__global__ void k_adam(AdamVec W, int nw, AdamVec B, int nb, uint16_t *__restrict__ p16, uint16_t *__restrict__ p16t,
+                       int in, float lr, float b1, float b2, float eps, float c1, float c2) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nw + nb) return;
+  const bool weight = i < nw;
+  if (!weight) i -= nw;
+  float *__restrict__ p = weight ? W.p : B.p;
+  const float *__restrict__ g = weight ? W.g : B.g;
+  float *__restrict__ m = weight ? W.m : B.m;
+  float *__restrict__ v = weight ? W.v : B.v;
   const float gi = g[i];
   const float mi = b1 * m[i] + (1.f - b1) * gi;
   const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
@@ -310,7 +323,14 @@ __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float
   v[i] = vi;
   const float pi = p[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
   p[i] = pi;
-  if (p16) p16[i] = f2bf(pi);
+  if (weight) {
+    const uint16_t h = f2bf(pi);
+    p16[i] = h;
+    if (in > 0) {
+      const int64_t t = chain::transposed_index(in, i);
+      if (t >= 0) p16t[t] = h;
+    }
+  }
 }
 
 __global__ void k_to_bf16(const float *__restrict__ a, uint16_t *__restrict__ b, int n) {
@@ -371,6 +391,28 @@ struct casl_mlp {
   std::vector<size_t> offA;
   int maxw = 0;
   int64_t step = 0;
+  // the fused training pass (mlp_chain.hpp): weights transposed, activations
+  // and gradients by feature, the batch's partial sums, the loss on the host
+  DevBuf<uint16_t> W16T, chain_act, chain_dz;
+  DevBuf<float> chain_cols, chain_loss;
+  PinnedBuf<float> host_loss;
+
+  // (10 .. 32)-128-128-128-128-1
+  bool chained() const {
+    return L == 5 && dim[0] <= chain::K0 && dim[1] == chain::H && dim[2] == chain::H && dim[3] == chain::H &&
+           dim[4] == chain::H && dim[5] == 1;
+  }
+  // uploads the transposed BF16 weights of host weights (layers concatenated)
+  void upload_transposed(const std::vector<uint16_t> &w16) {
+    if (!chained()) return;
+    std::vector<uint16_t> t(size_t(chain::TRANSPOSED_SIZE), 0);
+    for (size_t i = 0; i < w16.size(); ++i) {
+      const int64_t k = chain::transposed_index(dim[0], int64_t(i));
+      if (k >= 0) t[size_t(k)] = w16[i];
+    }
+    W16T.ensure(t.size());
+    HIP_CHECK(hipMemcpy(W16T.p, t.data(), t.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  }
 
   void ensure_cap(int n) {
     if (n <= cap) return;
@@ -404,6 +446,68 @@ void forward(casl_mlp *m, const float *x, int n, float *out, hipStream_t s) {
     gemm<false, false>(n, o, in, A, in, m->W16.p + m->offW[l], o, m->b.p + m->offb[l], nullptr, 0, last ? 0 : 1,
                        last ? out : nullptr, last ? nullptr : m->act16.p + m->offA[l + 1], o, s);
   }
+}
+
+// Forward, loss and all gradients of a (10 .. 32)-128x4-1 network in three
+// launches (the layer by layer pass takes 43): the chain keeps 32 samples'
+// activations in a wave's registers, one launch makes every layer's weight
+// gradients, one sums them.  Same bits as the layer by layer pass, the loss
+// aside (its sum there depends on the order of atomics).
+void chain_backward(casl_mlp *m, const float *x, const float *t, int n, bool want_loss, hipStream_t s) {
+  const int blocks64 = (n + 63) / 64, nb = (n + 31) / 32;
+  const int sp = k_splits(chain::H, chain::H, n);
+  const uint32_t nw = uint32_t(m->W.n);
+  m->chain_act.ensure(size_t(m->dim[0] + 4 * chain::H) * 64 * blocks64);
+  m->chain_dz.ensure(size_t(chain::COLS) * 64 * blocks64);
+  m->chain_cols.ensure(size_t(nb) * chain::COLS);
+  m->chain_loss.ensure(size_t(nb));
+  m->part.ensure(size_t(sp) * nw);
+  m->host_loss.ensure(1);
+  chain::TrainArgs a{};
+  a.x = x;
+  a.t = t;
+  a.n = n;
+  a.in = m->dim[0];
+  a.scale = 1.f / float(n);
+  a.mean = m->mean.p;
+  a.inv_std = m->inv_std.p;
+  a.W16 = m->W16.p;
+  a.W16T = m->W16T.p;
+  a.b = m->b.p;
+  a.act = m->chain_act.p;
+  a.dz = m->chain_dz.p;
+  a.colpart = m->chain_cols.p;
+  a.losspart = m->chain_loss.p;
+  chain::GradArgs g{};
+  g.act = a.act;
+  g.dz = a.dz;
+  g.n = n;
+  g.in = a.in;
+  // chunks as gemm() cuts them
+  g.kc = sp > 1 ? ((n + sp - 1) / sp + 15) / 16 * 16 : n;
+  g.nw = nw;
+  g.chunks = sp;
+  g.part = m->part.p;
+  prof_begin("k_train_chain", s);
+  hipLaunchKernelGGL(chain::k_train_chain, dim3(unsigned(blocks64)), dim3(chain::TRAIN_BLOCK), 0, s, a);
+  prof_end("k_train_chain", s);
+  prof_begin("k_train_grads", s);
+  hipLaunchKernelGGL(chain::k_train_grads, dim3(chain::grad_blocks(sp)), dim3(256), 0, s, g);
+  prof_end("k_train_grads", s);
+  chain::SumArgs u{};
+  u.part = m->part.p;
+  u.colpart = a.colpart;
+  u.losspart = a.losspart;
+  u.splits = sp;
+  u.nb = nb;
+  u.nw = nw;
+  u.wblocks = (nw + chain::SUM_BLOCK - 1) / chain::SUM_BLOCK;
+  u.gW = m->gW.p;
+  u.gb = m->gb.p;
+  u.loss = m->loss.p;
+  u.host_loss = want_loss ? m->host_loss.p : nullptr;
+  hipLaunchKernelGGL(chain::k_train_sums, dim3(u.wblocks + chain::COLS + 1), dim3(chain::SUM_BLOCK), 0, s, u);
+  HIP_CHECK(hipGetLastError());
 }
 
 // ------------------------------------------------ fused network curvature
@@ -603,6 +707,7 @@ int casl_mlp_create(const int32_t *dims, int n_layers, uint64_t seed, casl_mlp_t
     HIP_CHECK(hipMemcpy(m->mean.p, mean.data(), mean.size() * 4, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(m->inv_std.p, inv.data(), inv.size() * 4, hipMemcpyHostToDevice));
     m->loss.ensure(1);
+    m->upload_transposed(w16);
     *out = m.release();
   });
 }
@@ -691,6 +796,7 @@ int casl_mlp_set_params(casl_mlp_t *m, const float *weights, const float *biases
     for (size_t i = 0; i < m->W.n; ++i) w16[i] = f2bf(weights[i]);
     HIP_CHECK(hipMemcpy(m->W.p, weights, m->W.n * 4, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(m->W16.p, w16.data(), m->W.n * 2, hipMemcpyHostToDevice));
+    m->upload_transposed(w16);
     HIP_CHECK(hipMemcpy(m->b.p, biases, m->b.n * 4, hipMemcpyHostToDevice));
   });
 }
@@ -718,6 +824,14 @@ int casl_mlp_backward(casl_mlp_t *m, const float *x, const float *t, int n, floa
     if (!m || !x || !t || n <= 0) throw std::invalid_argument("bad arguments");
     if (m->dim[m->L] != 1) throw std::invalid_argument("training needs a scalar output");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (m->chained()) {
+      chain_backward(m, x, t, n, loss != nullptr, s);
+      if (loss) {
+        HIP_CHECK(hipStreamSynchronize(s));
+        *loss = *m->host_loss.p / float(n);
+      }
+      return;
+    }
     m->ensure_cap(n);  // sizes y32 before its address is taken
     forward(m, x, n, m->y32.p, s);
     hipLaunchKernelGGL(k_zero_f, dim3(1), dim3(64), 0, s, m->loss.p, 1);
@@ -772,10 +886,9 @@ int casl_mlp_adam_step(casl_mlp_t *m, float lr, float beta1, float beta2, float 
     const float c1 = float(1.0 / (1.0 - std::pow(double(beta1), double(m->step))));
     const float c2 = float(1.0 / (1.0 - std::pow(double(beta2), double(m->step))));
     const int nw = int(m->W.n), nb = int(m->b.n);
-    hipLaunchKernelGGL(k_adam, dim3(blocks(nw)), dim3(256), 0, s, m->W.p, m->gW.p, m->mW.p, m->vW.p, m->W16.p, nw,
-                       lr, beta1, beta2, eps, c1, c2);
-    hipLaunchKernelGGL(k_adam, dim3(blocks(nb)), dim3(256), 0, s, m->b.p, m->gb.p, m->mb.p, m->vb.p,
-                       (uint16_t *)nullptr, nb, lr, beta1, beta2, eps, c1, c2);
+    const AdamVec w{m->W.p, m->gW.p, m->mW.p, m->vW.p}, b{m->b.p, m->gb.p, m->mb.p, m->vb.p};
+    hipLaunchKernelGGL(k_adam, dim3(blocks(nw + nb)), dim3(256), 0, s, w, nw, b, nb, m->W16.p, m->W16T.p,
+                       m->chained() ? m->dim[0] : 0, lr, beta1, beta2, eps, c1, c2);
     HIP_CHECK(hipGetLastError());
   });
 }
