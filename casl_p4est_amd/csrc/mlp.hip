@@ -31,7 +31,6 @@ using namespace casl;
 using casl::dev::curv_hybrid2;
 using casl::dev::curv_hybrid3;
 using casl::dev::curv_normalize2;
-using casl::dev::curv_normalize3;
 
 namespace {
 
@@ -512,145 +511,233 @@ void chain_backward(casl_mlp *m, const float *x, const float *t, int n, bool wan
 
 // ------------------------------------------------ fused network curvature
 // The learned h*kappa of samples in one launch: input normalisation, every
-// layer of a (10|28)-128-128-128-128-1 network on MFMA with the activations
-// in LDS, and the hybrid blend.  Each block holds all weights in LDS (stored
-// [out][in], so a column's 8 consecutive k are one 16-byte read) and runs
-// tiles of 128 network rows: 2D samples give 2 rows each (as is, reflected),
-// 3D samples one.  Wave w owns rows 32w .. 32w + 31 in every layer: it reads
-// only its own rows of X and overwrites them with the layer's output, so the
-// layers need no barrier.  Every product, bias add, ReLU and BF16 rounding is
-// the one k_gemm makes, in the same order (the K loop ascends in steps of
-// 16), so the result equals casl_curvature_normalize(_3d) + casl_mlp_forward
-// + casl_curvature_hybrid(_3d) bit for bit.
-constexpr int NF_H = 128;            // hidden width
-constexpr int NF_XS = NF_H + 8;      // LDS row stride (halves) of X and of the hidden weights
-constexpr int NF_K0S = 32 + 8;       // LDS row stride of the first layer's weights
-constexpr int NF_ROWS = 128;         // network rows per tile
-
+// layer of a (10|28)-128-128-128-128-1 network on MFMA with the activations in
+// registers (mlp_chain.hpp), and the hybrid blend.  A block holds all weights
+// in LDS, copied once; each of its eight waves then runs 64 network rows at a
+// time by itself, two blocks of 32 that share every weight operand it reads
+// (one block of 32 would need the LDS's whole bandwidth to feed the MFMAs).  2D
+// samples give 2 rows each (as is, reflected), 3D samples one.  Every product,
+// bias add, ReLU and BF16 rounding is the one k_gemm makes, in the same order
+// (the K loop ascends in steps of 16), so the result equals
+// casl_curvature_normalize(_3d) + casl_mlp_forward + casl_curvature_hybrid(_3d)
+// bit for bit.  3.3M samples: 1.36 ms in 3D and 2.26 ms in 2D with activations in
+// LDS and one wave per SIMD, 0.50 and 0.75 ms (890 TFLOP/s) here.
 struct FusedNet {
-  const uint16_t *W16;  // [in][out] per layer, concatenated
-  const float *b;       // per layer, concatenated
+  const uint16_t *W16T;  // transposed layers (mlp_chain.hpp)
+  const uint16_t *W4;    // the last layer's 128 weights
+  const float *b;        // per layer, concatenated
   const float *mean, *inv_std;
-  size_t offW[5], offb[5];
-  int in;               // 10 or 28
 };
+constexpr int NF_BLOCK = 512, NF_WAVES = NF_BLOCK / 64;
+constexpr int NF_ROWS = 64;  // network rows of a wave at a time
+constexpr int NF_FS = 28;    // LDS row stride of a wave's 32 samples' features (3D)
 
-// LDS footprint (bytes): weights, X, biases, predictions
-constexpr size_t NF_LDS = size_t(NF_H) * NF_K0S * 2 + 3 * size_t(NF_H) * NF_XS * 2 + size_t(32) * NF_XS * 2 +
-                          size_t(NF_ROWS) * NF_XS * 2 + (4 * NF_H + 1) * 4 + NF_ROWS * 4;
-static_assert(NF_LDS <= 160 * 1024, "fused network kernel exceeds the LDS of a compute unit");
+struct NetLds {
+  uint16_t W0[chain::H * chain::W0S];
+  uint16_t Wh[3][chain::H * chain::WS];
+  uint16_t W4[chain::H];
+  float bias[4 * chain::H];
+  float mean[chain::K0], inv_std[chain::K0];
+  float feat[NF_WAVES][32 * NF_FS];
+};
+static_assert(sizeof(NetLds) <= 160 * 1024, "fused network kernel exceeds the LDS of a compute unit");
+
+// k_pack_input's rounding of the eight inputs o[v] from input k0 on (lds: the
+// scaler), as one MFMA operand half; inputs past `in` are zero
+__device__ __forceinline__ chain::bf16x8 pack_inputs(const NetLds &lds, const float (&o)[8], int k0, int in,
+                                                     bool valid) {
+  chain::u32x4 w;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    float f[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int k = k0 + 2 * v + q;
+      f[q] = (valid && k < in) ? (o[2 * v + q] - lds.mean[k]) * lds.inv_std[k] : 0.f;
+    }
+    w[v] = chain::pack_bf16(f[0], f[1]);
+  }
+  return __builtin_bit_cast(chain::bf16x8, w);
+}
+
+// The inputs of 3D sample li of the 32 whose features lie at f (curv_normalize3,
+// the same operations on the values this half of the wave needs): new axis b
+// reads old axis p[b] reflected by r, so value (i, j, k) of the canonical
+// orientation is feature 13 + i S0 + j S1 + k S2 with S_b = r stride(p[b]).
+__device__ __forceinline__ void inputs3(const NetLds &lds, const float *__restrict__ f, bool valid, int hh,
+                                        chain::bf16x8 *op) {
+  const float sg = f[27] > 0.f ? -1.f : 1.f;
+  float g[3];
+  int S[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    constexpr int stride[3] = {9, 3, 1};
+    g[a] = f[13 + stride[a]] * sg - f[13 - stride[a]] * sg;
+    if (g[a] == 0.f) g[a] = float(dev::EPS);
+    S[a] = g[a] < 0.f ? -stride[a] : stride[a];
+    g[a] = fabsf(g[a]);
+  }
+  auto swap_if = [&](int a, int b, bool c) {
+    const float x = g[a], y = g[b];
+    g[a] = c ? y : x;
+    g[b] = c ? x : y;
+    const int u = S[a], v = S[b];
+    S[a] = c ? v : u;
+    S[b] = c ? u : v;
+  };
+  swap_if(0, 1, g[1] > g[0]);
+  const bool last = g[2] > g[1];
+  swap_if(1, 2, last);
+  swap_if(0, 1, last && g[1] > g[0]);
+  const float f0 = f[13] * sg;
+  const float gx = 0.5f * (f[13 + S[0]] * sg - f[13 - S[0]] * sg);
+  const float gy = 0.5f * (f[13 + S[1]] * sg - f[13 - S[1]] * sg);
+  const float gz = 0.5f * (f[13 + S[2]] * sg - f[13 - S[2]] * sg);
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    float o[8];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      // input q of this half: its place in the cube is known for each half
+      float c[3];
+      int at = 13;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const int q0 = 16 * ks + v, q1 = q0 + 8, d = a == 0 ? 9 : (a == 1 ? 3 : 1);
+        const int c0 = (q0 / d) % 3 - 1, c1 = (q1 / d) % 3 - 1;
+        c[a] = hh ? float(c1) : float(c0);
+        at += hh ? c1 * S[a] : c0 * S[a];
+      }
+      const int q0 = 16 * ks + v, q1 = q0 + 8;
+      const bool cube = q1 < 27 || (q0 < 27 && !hh);
+      const float x = cube ? f[at] * sg : 0.f;
+      o[v] = x - (f0 + (c[0] * gx + c[1] * gy + c[2] * gz));
+      if (q0 == 4) o[v] = hh ? (q1 == 12 ? gz : o[v]) : gx;  // inputs 4 and 12
+      if (q1 == 10) o[v] = hh ? gy : o[v];
+      if (q1 == 13) o[v] = hh ? f0 : o[v];
+      if (q1 == 27) o[v] = hh ? f[27] * sg : o[v];
+    }
+    op[ks] = pack_inputs(lds, o, 16 * ks + 8 * hh, 28, valid);
+  }
+}
 
 template <int D>
-__global__ void __launch_bounds__(256)
-    k_net_curvature(FusedNet net, const float *__restrict__ feat, int64_t n, float lo, float hi, int residual,
+__global__ void __launch_bounds__(NF_BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    k_net_curvature(FusedNet net, const float *__restrict__ feat, int wide, int64_t n, float lo, float hi, int residual,
                     float dead, float *__restrict__ hk) {
-  constexpr int NFEAT = D == 2 ? 10 : 28;                 // features per sample
-  constexpr int RPS = D == 2 ? 2 : 1;                     // network rows per sample
-  constexpr int SPT = NF_ROWS / RPS;                      // samples per tile
-  extern __shared__ __align__(16) unsigned char lds[];
-  uint16_t *W0 = reinterpret_cast<uint16_t *>(lds);                 // [128][NF_K0S]
-  uint16_t *Wh = W0 + NF_H * NF_K0S;                                // 3 x [128][NF_XS]
-  uint16_t *W4 = Wh + 3 * NF_H * NF_XS;                             // [32][NF_XS], row 0 = last layer
-  uint16_t *X = W4 + 32 * NF_XS;                                    // [128][NF_XS]
-  float *bias = reinterpret_cast<float *>(X + NF_ROWS * NF_XS);     // 4 x 128 + 1
-  float *pred = bias + 4 * NF_H + 1;                                // [128]
-  const int tid = int(threadIdx.x), wave = tid >> 6, lane = tid & 63;
-  const int in = net.in, k0p = (in + 15) / 16 * 16;
-  // weights, transposed into [out][in], zero beyond each layer's width
-  for (int e = tid; e < NF_H * 32; e += 256) {
-    const int j = e / 32, k = e % 32;
-    W0[j * NF_K0S + k] = k < in ? net.W16[net.offW[0] + size_t(k) * NF_H + j] : uint16_t(0);
+  using namespace chain;
+  constexpr int NFEAT = D == 2 ? 10 : 28;  // features per sample
+  constexpr int RPS = D == 2 ? 2 : 1;      // network rows per sample
+  constexpr int BS32 = 32 / RPS;           // samples of a block of 32 rows
+  constexpr int KS0 = D == 2 ? 1 : 2;      // first layer's steps of 16
+  extern __shared__ __align__(16) unsigned char raw[];
+  NetLds &lds = *reinterpret_cast<NetLds *>(raw);
+  const int tid = int(threadIdx.x), wave = tid >> 6, lane = tid & 63, li = lane & 31, hh = lane >> 5;
+  // weights, 16 bytes at a time
+  for (int c = tid; c < H * K0 / 8; c += NF_BLOCK)
+    *reinterpret_cast<u32x4 *>(lds.W0 + (c >> 2) * W0S + (c & 3) * 8) = reinterpret_cast<const u32x4 *>(net.W16T)[c];
+  for (int c = tid; c < 3 * H * H / 8; c += NF_BLOCK) {
+    const int l = c / (H * H / 8), e = c % (H * H / 8);
+    *reinterpret_cast<u32x4 *>(lds.Wh[l] + (e >> 4) * WS + (e & 15) * 8) =
+        reinterpret_cast<const u32x4 *>(net.W16T + H * K0)[c];
   }
-  for (int l = 1; l <= 3; ++l)
-    for (int e = tid; e < NF_H * NF_H; e += 256) {
-      const int k = e / NF_H, j = e % NF_H;  // coalesced over j in global memory
-      Wh[(l - 1) * NF_H * NF_XS + j * NF_XS + k] = net.W16[net.offW[l] + size_t(k) * NF_H + j];
-    }
-  for (int e = tid; e < 32 * NF_H; e += 256) {
-    const int j = e / NF_H, k = e % NF_H;
-    W4[j * NF_XS + k] = j == 0 ? net.W16[net.offW[4] + size_t(k)] : uint16_t(0);
+  if (tid < H) lds.W4[tid] = net.W4[tid];
+  lds.bias[tid] = net.b[tid];
+  if (tid < NFEAT) {
+    lds.mean[tid] = net.mean[tid];
+    lds.inv_std[tid] = net.inv_std[tid];
   }
-  for (int e = tid; e < 4 * NF_H + 1; e += 256) {
-    const int l = e / NF_H, j = e % NF_H;
-    bias[e] = net.b[net.offb[l] + size_t(j)];
-  }
-  const int64_t ntiles = (n + SPT - 1) / SPT;
-  const int li = lane & 31, lk = (lane >> 5) * 8;
-  const int row0 = wave * 32;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    __syncthreads();  // weights loaded; the previous tile's X and pred consumed
-    // inputs: normalised, standardised, BF16 (k_pack_input's rounding)
-    for (int t = tid; t < SPT; t += 256) {
-      const int64_t smp = tile * SPT + t;
-      float o[RPS * NFEAT];
-      if (smp < n) {
-        if constexpr (D == 2)
+  const float b4 = net.b[4 * H];
+  __syncthreads();
+  float *fw = lds.feat[wave];
+  const int64_t ntiles = (n * RPS + NF_ROWS - 1) / NF_ROWS;
+  for (int64_t tile = int64_t(wave) * gridDim.x + blockIdx.x; tile < ntiles; tile += int64_t(NF_WAVES) * gridDim.x) {
+    bf16x8 op[2][8];
+    float ihk[2];
+#pragma unroll
+    for (int blk = 0; blk < 2; ++blk) {
+      const int64_t s0 = (tile * 2 + blk) * BS32, smp = s0 + li / RPS;
+      const bool valid = smp < n;
+      if constexpr (D == 3) {
+        // the 32 samples' features through LDS, then each half's inputs
+        wave_order();
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int c = lane + 64 * h;  // 224 pieces of four
+          if (c < 32 * NFEAT / 4 && s0 * NFEAT + 4 * c < n * NFEAT) {
+            const float *src = feat + s0 * NFEAT + 4 * c;
+            float4 v;
+            if (wide) {
+              v = *reinterpret_cast<const float4 *>(src);
+            } else {
+              v.x = src[0];
+              v.y = src[1];
+              v.z = src[2];
+              v.w = src[3];
+            }
+            *reinterpret_cast<float4 *>(fw + 4 * c) = v;
+          }
+        }
+        wave_order();
+        ihk[blk] = fw[li * NF_FS + 27];
+        inputs3(lds, fw + li * NF_FS, valid, hh, op[blk]);
+      } else {
+        float o[20];
+#pragma unroll
+        for (int q = 0; q < 20; ++q) o[q] = 0.f;
+        ihk[blk] = 0.f;
+        if (valid) {
           curv_normalize2(feat + NFEAT * smp, o);
-        else
-          curv_normalize3(feat + NFEAT * smp, o);
-      }
+          ihk[blk] = feat[NFEAT * smp + 9];
+        }
+        const bool refl = (li & 1) != 0;
+        float x[8];
 #pragma unroll
-      for (int r = 0; r < RPS; ++r) {
-        uint16_t *xr = X + (t * RPS + r) * NF_XS;
-        for (int k = 0; k < 32; ++k)
-          xr[k] = (smp < n && k < in) ? f2bf((o[r * NFEAT + k] - net.mean[k]) * net.inv_std[k]) : uint16_t(0);
+        for (int v = 0; v < 8; ++v) {
+          const float a = refl ? o[10 + v] : o[v];
+          const float b = v < 2 ? (refl ? o[18 + v] : o[8 + v]) : 0.f;
+          x[v] = hh ? b : a;
+        }
+        op[blk][0] = pack_inputs(lds, x, 8 * hh, NFEAT, valid);
       }
+      __builtin_amdgcn_sched_barrier(0);  // keeps one block's inputs from living beside the next one's
     }
-    __syncthreads();
-    // hidden layers: wave-owned rows, in place
+    // hidden layers, 32 features at a time
+    Packed<4> out[2];
+#pragma unroll
     for (int l = 0; l < 4; ++l) {
-      const uint16_t *W = l == 0 ? W0 : Wh + (l - 1) * NF_H * NF_XS;
-      const int ws = l == 0 ? NF_K0S : NF_XS;
-      const int K = l == 0 ? k0p : NF_H;
-      f32x16 acc[4];
+      const uint16_t *W = l == 0 ? lds.W0 : lds.Wh[l - 1];
+      const int KS = l == 0 ? KS0 : 8, S = l == 0 ? W0S : WS;
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int rb = 0; rb < 4; ++rb) {
+        f32x16 c[2];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[c][r] = 0.f;
-      for (int k0 = 0; k0 < K; k0 += 16) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(X + (row0 + li) * NF_XS + k0 + lk);
+        for (int r = 0; r < 16; ++r) c[0][r] = c[1][r] = 0.f;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const bf16x8 b = *reinterpret_cast<const bf16x8 *>(W + (32 * c + li) * ws + k0 + lk);
-          acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[c], 0, 0, 0);
+        for (int ks = 0; ks < KS; ++ks) {
+          const bf16x8 a = *reinterpret_cast<const bf16x8 *>(W + (32 * rb + li) * S + ks * 16 + hh * 8);
+          c[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, op[0][ks], c[0], 0, 0, 0);
+          c[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, op[1][ks], c[1], 0, 0, 0);
         }
+        bias_relu(c[0], lds.bias + l * H + 32 * rb, lane, out[0].p[rb]);
+        bias_relu(c[1], lds.bias + l * H + 32 * rb, lane, out[1].p[rb]);
       }
-      const float *bl = bias + l * NF_H;
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), col = 32 * c + li;
-          float v = acc[c][r];
-          v += bl[col];
-          v = v > 0.f ? v : 0.f;
-          X[row * NF_XS + col] = f2bf(v);
-        }
+        for (int ks = 0; ks < 8; ++ks) op[blk][ks] = operand(out[blk], ks);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // last layer (one output column)
-    {
-      f32x16 acc;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-      for (int k0 = 0; k0 < NF_H; k0 += 16) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(X + (row0 + li) * NF_XS + k0 + lk);
-        const bf16x8 b = *reinterpret_cast<const bf16x8 *>(W4 + li * NF_XS + k0 + lk);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+    for (int blk = 0; blk < 2; ++blk) {
+      const float y = last_output(op[blk], lds.W4, lane) + b4;  // rows in lanes 0 .. 31
+      const int64_t smp = (tile * 2 + blk) * BS32 + li / RPS;
+      if constexpr (D == 2) {
+        const float y1 = __shfl_down(y, 1);
+        if (hh == 0 && (li & 1) == 0 && smp < n) hk[smp] = curv_hybrid2(ihk[blk], y, y1, lo, hi, residual);
+      } else {
+        if (hh == 0 && smp < n) hk[smp] = curv_hybrid3(ihk[blk], y, lo, hi, residual, dead);
       }
-      if (li == 0) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) pred[row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)] = acc[r] + bias[4 * NF_H];
-      }
-    }
-    __syncthreads();
-    for (int t = tid; t < SPT; t += 256) {
-      const int64_t smp = tile * SPT + t;
-      if (smp >= n) continue;
-      const float ihk = feat[NFEAT * smp + NFEAT - 1];
-      if constexpr (D == 2)
-        hk[smp] = curv_hybrid2(ihk, pred[2 * t], pred[2 * t + 1], lo, hi, residual);
-      else
-        hk[smp] = curv_hybrid3(ihk, pred[t], lo, hi, residual, dead);
     }
   }
 }
@@ -717,39 +804,35 @@ int casl_curvature_learned(casl_mlp_t *m, const float *feat, int64_t n, float lo
   return guarded([&]() {
     if (!m || n < 0 || (n > 0 && (!feat || !hk)) || !(hi > lo) || !(lo >= 0.f) || !(deadband >= 0.f))
       throw std::invalid_argument("bad arguments");
-    if (m->L != 5 || (m->dim[0] != 10 && m->dim[0] != 28) || m->dim[1] != NF_H || m->dim[2] != NF_H ||
-        m->dim[3] != NF_H || m->dim[4] != NF_H || m->dim[5] != 1)
+    if (m->L != 5 || (m->dim[0] != 10 && m->dim[0] != 28) || !m->chained())
       throw std::invalid_argument("casl_curvature_learned takes a (10|28)-128-128-128-128-1 network");
     if (n == 0) return;
     FusedNet net{};
-    net.W16 = m->W16.p;
+    net.W16T = m->W16T.p;
+    net.W4 = m->W16.p + m->offW[4];
     net.b = m->b.p;
     net.mean = m->mean.p;
     net.inv_std = m->inv_std.p;
-    for (int l = 0; l < 5; ++l) {
-      net.offW[l] = m->offW[l];
-      net.offb[l] = m->offb[l];
-    }
-    net.in = m->dim[0];
     hipStream_t s = static_cast<hipStream_t>(stream);
     int dev = 0, cus = 0;
     HIP_CHECK(hipGetDevice(&dev));
     HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int64_t spt = net.in == 10 ? NF_ROWS / 2 : NF_ROWS;
-    const int64_t ntiles = (n + spt - 1) / spt;
+    // a wave per 64 rows, one block per compute unit; few rows spread over the
+    // units before they share one
+    const int64_t ntiles = (n * (m->dim[0] == 10 ? 2 : 1) + NF_ROWS - 1) / NF_ROWS;
     const unsigned grid = unsigned(std::max<int64_t>(1, std::min<int64_t>(ntiles, int64_t(cus))));
+    const int wide = (reinterpret_cast<uintptr_t>(feat) & 15) == 0;
     prof_begin("k_net_curvature", s);
-    if (net.in == 10) {
-      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_net_curvature<2>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(NF_LDS)));
-      hipLaunchKernelGGL(k_net_curvature<2>, dim3(grid), dim3(256), NF_LDS, s, net, feat, n, lo, hi, residual,
+    auto launch = [&](auto kernel) {
+      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(sizeof(NetLds))));
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(NF_BLOCK), sizeof(NetLds), s, net, feat, wide, n, lo, hi, residual,
                          deadband, hk);
-    } else {
-      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_net_curvature<3>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(NF_LDS)));
-      hipLaunchKernelGGL(k_net_curvature<3>, dim3(grid), dim3(256), NF_LDS, s, net, feat, n, lo, hi, residual,
-                         deadband, hk);
-    }
+    };
+    if (m->dim[0] == 10)
+      launch(&k_net_curvature<2>);
+    else
+      launch(&k_net_curvature<3>);
     prof_end("k_net_curvature", s);
     HIP_CHECK(hipGetLastError());
   });
