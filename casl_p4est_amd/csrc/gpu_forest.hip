@@ -736,8 +736,7 @@ int casl_device_grid_stencil(const casl_device_grid_t *g, casl_stencil_t **out) 
     tab.wall = g->wall.p;
     tab.zero_distance_threshold = g->zdt;
     auto st = std::make_unique<casl_stencil>();
-    upload_device_tables(tab, st.get(), nullptr);
-    build_tiles_device(tab, st.get(), nullptr);
+    stencil_from_device_tables(tab, st.get(), nullptr);
     HIP_CHECK(hipStreamSynchronize(nullptr));
     *out = st.release();
   });

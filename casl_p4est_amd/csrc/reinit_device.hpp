@@ -575,10 +575,9 @@ void upload_tile_host(const TileHost &H, int64_t n_nodes, casl_stencil *st);
 
 // Grid-wide tables of a stencil from tables already on the device (checked
 // there, distances converted to FP32 exactly), and the tiled encoding built
-// on the device (tiles_gpu.hip); on failure the latter leaves the stencil on
+// on the device (tiles_gpu.hip); where there is none the stencil stays on
 // the two-pass path with the reason in tile_error.
-void upload_device_tables(const casl_flat_stencil &dtab, casl_stencil *st, hipStream_t s);
-void build_tiles_device(const casl_flat_stencil &dtab, casl_stencil *st, hipStream_t s);
+void stencil_from_device_tables(const casl_flat_stencil &dtab, casl_stencil *st, hipStream_t s);
 
 // A reinitialization call (casl_reinit's arguments, no mask) whose buffers are
 // carved from [base, base + cap) instead of the stencil's own scratch:
