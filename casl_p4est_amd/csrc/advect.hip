@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(BLOCK) k_advect(TB t, const double *__restrict
 // T u H1, then advect_value for T.  out = result, or (RK_AVG) out = (out +
 // result) / 2.  The loads a node needs (its record, slot and vn, and the
 // value being averaged) are issued before the first barrier.
-template <int D, bool RK_AVG, bool WT, bool SMALL>
+template <int D, bool RK_AVG, int CELLS, bool SMALL>
 __global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
     __attribute__((amdgpu_waves_per_eu((tile_waves<D, double, SMALL>()))))
     k_tile_advect(TileArgs<double> A, const double *__restrict__ vn, double dt) {
@@ -64,7 +64,7 @@ __global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
   TileCtx<D> c;
   c.load(A, tile);
   const int s = c.s, nT = c.nT, hb = c.hb, nH = c.nH, nH1 = c.nH1;
-  const bool ufast = A.geom.template uni_fast<WT>();
+  const bool ufast = A.geom.template uni_fast<CELLS>();
   RecRegs trec[KT];
   int tslot[KT];
 #pragma unroll
@@ -78,12 +78,12 @@ __global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
 #pragma unroll
   for (int k = 0; k < KT; ++k) {
     const int i = int(threadIdx.x) + k * BT;
-    if (i < nT) tile_pass_a<D, double, WT, SMALL>(A, c, ufast, trec[k], tslot[k], i, phis, dds);
+    if (i < nT) tile_pass_a<D, double, CELLS, SMALL>(A, c, ufast, trec[k], tslot[k], i, phis, dds);
   }
   for (int i = nT + int(threadIdx.x); i < nT + nH1; i += BT) {
     RecRegs r;
     const int js = fetch_record<D>(A, c, i, r);
-    tile_pass_a<D, double, WT, SMALL>(A, c, ufast, r, js, i, phis, dds);
+    tile_pass_a<D, double, CELLS, SMALL>(A, c, ufast, r, js, i, phis, dds);
   }
   __syncthreads();
 #pragma unroll
@@ -93,18 +93,18 @@ __global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
     int j = tslot[k];
     double r;
     if (ufast && c.uniform(i)) {
-      UniStencil<D, double, WT> st;
+      UniStencil<D, double, CELLS> st;
       j = st.load(trec[k].w, A.geom);
       r = advect_value<D>(st, j, 0, vn[s + j], dt, phis, dds, DMAX);
     } else {
       const TileRec rec = record_at<D>(c, i, trec[k], j);
       const uint8_t w = uint8_t((rec.geo >> 24) & 63u);
       if (!(rec.geo & GEO_IRREGULAR)) {
-        RegStencil<D, double, WT> st;
+        RegStencil<D, double, CELLS> st;
         st.load(rec, A.geom);
         r = advect_value<D>(st, j, w, vn[s + j], dt, phis, dds, DMAX);
       } else {
-        HangStencil<D, double, WT> st;
+        HangStencil<D, double, CELLS> st;
         st.load(rec, c.ext_of(A.ext, i), A.geom);
         r = advect_value<D>(st, j, w, vn[s + j], dt, phis, dds, DMAX);
       }
@@ -153,15 +153,24 @@ void run_advect(casl_stencil *st, double *phi, const double *vn, const double *v
       ta.phin = in;
       ta.out = out;
       prof_begin("k_tile_advect", s);
-      auto launch = [&](auto wt, auto small) {
+      auto launch = [&](auto cells, auto small) {
         constexpr bool SM = decltype(small)::value;
-        hipLaunchKernelGGL((k_tile_advect<D, decltype(rk)::value, decltype(wt)::value, SM>), g,
+        hipLaunchKernelGGL((k_tile_advect<D, decltype(rk)::value, decltype(cells)::value, SM>), g,
                            dim3(tile_block<D, double, SM>()), 0, s, ta, v, dt);
       };
-      if (st->weighted_tiles())
-        st->small ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{});
-      else
-        st->small ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{});
+      auto of_size = [&](auto cells) {
+        st->small ? launch(cells, std::true_type{}) : launch(cells, std::false_type{});
+      };
+      switch (tile_cells(st, true)) {
+        case DYADIC_CUBES:
+          of_size(std::integral_constant<int, DYADIC_CUBES>{});
+          break;
+        case WEIGHTED_CUBES:
+          of_size(std::integral_constant<int, WEIGHTED_CUBES>{});
+          break;
+        default:
+          of_size(std::integral_constant<int, ANY_CELLS>{});
+      }
       prof_end("k_tile_advect", s);
     };
     stage(std::false_type{}, phi, st->phi0.p, vn);

@@ -156,7 +156,7 @@ constexpr int batch_waves() {
 
 // Persistent kernel over trees whose pseudo-time stages run tile by tile in
 // LDS; every tree's result is its single-tree tiled result.
-template <int D, class R, int BLOCK>
+template <int D, class R, int BLOCK, int CELLS>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(batch_waves<R, BLOCK>())))
     k_batch_tiles(BatchTileArgs<R> A) {
   __shared__ R phis[TileLimits<D>::LMAX];
@@ -177,13 +177,13 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(batc
       a.phin = A.cur;
       a.out = A.nxt;
       for (int tile = t0; tile < t1; ++tile) {
-        tile_stage<D, R, true, false, BLOCK>(a, tile, phis, dds);
+        tile_stage<D, R, true, false, BLOCK, CELLS>(a, tile, phis, dds);
         __syncthreads();
       }
       a.phin = A.nxt;
       a.out = A.cur;
       for (int tile = t0; tile < t1; ++tile) {
-        tile_stage<D, R, true, true, BLOCK>(a, tile, phis, dds);
+        tile_stage<D, R, true, true, BLOCK, CELLS>(a, tile, phis, dds);
         __syncthreads();
       }
     }
@@ -226,12 +226,12 @@ constexpr bool tile_block_ok(int block) {
   return block == 512 || (D == 2 && (block == 256 || block == 1024));
 }
 
-template <int D, class R>
+template <int D, class R, int CELLS>
 TileKernelFn<D, R> pick_tile_kernel(int block) {
-  if (block == 512) return &k_batch_tiles<D, R, 512>;
+  if (block == 512) return &k_batch_tiles<D, R, 512, CELLS>;
   if constexpr (D == 2) {
-    if (block == 256) return &k_batch_tiles<D, R, 256>;
-    if (block == 1024) return &k_batch_tiles<D, R, 1024>;
+    if (block == 256) return &k_batch_tiles<D, R, 256, CELLS>;
+    if (block == 1024) return &k_batch_tiles<D, R, 1024, CELLS>;
   }
   throw std::invalid_argument("unsupported tiled batch block size");
 }
@@ -329,10 +329,19 @@ void launch_batch(casl_batch *B, double *phi, int n_iter, hipStream_t s, bool al
     // flags and s_fix of every tree in tile-record order (FP64 tiled prep)
     TileArgs<double> tp = tile_args<double>(&st);
     tp.phin = st.phi0.p;
-    hipLaunchKernelGGL((k_tile_prep<D, R, true>), dim3(unsigned(st.n_tiles)), dim3(TILE_BLOCK_F64), 0, s, tp,
-                       (const uint8_t *)nullptr, -DBL_MAX, DBL_MAX, st.zdt, st.flags.p, A.sfix);
+    const bool cubes = tile_cells(&st, sizeof(R) == 8) == DYADIC_CUBES;
+    auto prep = [&](auto cells) {
+      hipLaunchKernelGGL((k_tile_prep<D, R, true, decltype(cells)::value>), dim3(unsigned(st.n_tiles)),
+                         dim3(TILE_BLOCK_F64), 0, s, tp, (const uint8_t *)nullptr, -DBL_MAX, DBL_MAX, st.zdt,
+                         st.flags.p, A.sfix);
+    };
+    if (cubes)
+      prep(std::integral_constant<int, DYADIC_CUBES>{});
+    else
+      prep(std::integral_constant<int, ANY_CELLS>{});
     HIP_CHECK(hipGetLastError());
-    TileKernelFn<D, R> fn = pick_tile_kernel<D, R>(B->sched.block);
+    TileKernelFn<D, R> fn = cubes ? pick_tile_kernel<D, R, DYADIC_CUBES>(B->sched.block)
+                                  : pick_tile_kernel<D, R, ANY_CELLS>(B->sched.block);
     int occ = 0;
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *)fn, B->sched.block, 0));
     occ = std::max(occ, 1);

@@ -244,18 +244,24 @@ ReinitSizes reinit_sizes(size_t N, bool so, bool tiled) {
   return z;
 }
 
-// fn(wt): wt is true for FP64 on a geometry that is not dyadic, where the
-// kernels keep the weighted form of regular faces; the mixed path's FP32
-// stages (and its prep) do not need it.
+// fn(cells): what the tiles' kernels know of the cells when compiled (Cells).
+// FP64 on cubic cells that are not dyadic keeps the weighted form of regular
+// faces; the mixed path's FP32 stages (and its prep) do not need it.
 template <class R, class Fn>
-void with_weights(bool weighted, Fn &&fn) {
-  if constexpr (sizeof(R) == 8) {
-    if (weighted) {
-      fn(std::true_type{});
+void with_cells(const casl_stencil *st, Fn &&fn) {
+  switch (tile_cells(st, sizeof(R) == 8)) {
+    case DYADIC_CUBES:
+      fn(std::integral_constant<int, DYADIC_CUBES>{});
       return;
-    }
+    case WEIGHTED_CUBES:
+      if constexpr (sizeof(R) == 8) {
+        fn(std::integral_constant<int, WEIGHTED_CUBES>{});
+        return;
+      }
+      [[fallthrough]];
+    default:
+      fn(std::integral_constant<int, ANY_CELLS>{});
   }
-  fn(std::false_type{});
 }
 
 // Every scratch buffer a reinitialization call of this kind uses, allocated
@@ -299,7 +305,7 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
   const bool so = order_space > 1;
   const unsigned grid = grid_for(N);
 
-  const bool tiled = st->use_tiles(sizeof(R) == 8), wt_tiles = st->weighted_tiles();
+  const bool tiled = st->use_tiles(sizeof(R) == 8);
   HIP_CHECK(hipMemcpyAsync(B.phi0, phi, sizeof(double) * N, hipMemcpyDeviceToDevice, s));
   if (so && !tiled) {
     prof_begin("k_dd", s);
@@ -323,16 +329,16 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
     tp.phin = B.phi0;
     const dim3 g(unsigned(st->n_tiles));
     prof_begin("k_tile_prep", s);
-    auto prep = [&](auto second, auto wt, auto small) {
+    auto prep = [&](auto second, auto cells, auto small) {
       constexpr bool SM = decltype(small)::value;
-      hipLaunchKernelGGL((k_tile_prep<D, R, decltype(second)::value, decltype(wt)::value, SM>), g,
+      hipLaunchKernelGGL((k_tile_prep<D, R, decltype(second)::value, decltype(cells)::value, SM>), g,
                          dim3(tile_block<D, double, SM>()), 0, s, tp, mask, lim_low, lim_high, st->zdt, B.flags, sfix);
     };
-    with_weights<R>(wt_tiles, [&](auto wt) {
+    with_cells<R>(st, [&](auto cells) {
       if (st->small)
-        so ? prep(std::true_type{}, wt, std::true_type{}) : prep(std::false_type{}, wt, std::true_type{});
+        so ? prep(std::true_type{}, cells, std::true_type{}) : prep(std::false_type{}, cells, std::true_type{});
       else
-        so ? prep(std::true_type{}, wt, std::false_type{}) : prep(std::false_type{}, wt, std::false_type{});
+        so ? prep(std::true_type{}, cells, std::false_type{}) : prep(std::false_type{}, cells, std::false_type{});
     });
     prof_end("k_tile_prep", s);
   } else {
@@ -391,18 +397,19 @@ void run_reinit(casl_stencil *st, double *phi, const uint8_t *mask, int order_sp
     ta.out = out;
     const dim3 g(unsigned(st->n_tiles));
     prof_begin("k_tile_stage", s);
-    auto launch = [&](auto second, auto rk, auto wt) {
-      constexpr bool SO = decltype(second)::value, RK = decltype(rk)::value, WT = decltype(wt)::value;
+    auto launch = [&](auto second, auto rk, auto cells) {
+      constexpr bool SO = decltype(second)::value, RK = decltype(rk)::value;
+      constexpr int CELLS = decltype(cells)::value;
       if (st->small)
-        hipLaunchKernelGGL((k_small_stage<D, R, SO, RK, WT>), g, dim3(tile_block<D, R, true>()), 0, s, ta);
+        hipLaunchKernelGGL((k_small_stage<D, R, SO, RK, CELLS>), g, dim3(tile_block<D, R, true>()), 0, s, ta);
       else
-        hipLaunchKernelGGL((k_tile_stage<D, R, SO, RK, WT>), g, dim3(tile_block<D, R, false>()), 0, s, ta);
+        hipLaunchKernelGGL((k_tile_stage<D, R, SO, RK, CELLS>), g, dim3(tile_block<D, R, false>()), 0, s, ta);
     };
-    with_weights<R>(wt_tiles, [&](auto wt) {
+    with_cells<R>(st, [&](auto cells) {
       if (so)
-        avg ? launch(std::true_type{}, std::true_type{}, wt) : launch(std::true_type{}, std::false_type{}, wt);
+        avg ? launch(std::true_type{}, std::true_type{}, cells) : launch(std::true_type{}, std::false_type{}, cells);
       else
-        avg ? launch(std::false_type{}, std::true_type{}, wt) : launch(std::false_type{}, std::false_type{}, wt);
+        avg ? launch(std::false_type{}, std::true_type{}, cells) : launch(std::false_type{}, std::false_type{}, cells);
     });
     prof_end("k_tile_stage", s);
   };

@@ -10,6 +10,18 @@
 namespace casl {
 namespace dev {
 
+// What a kernel knows of its tiles' cells when it is compiled.  DYADIC_CUBES
+// drops the per-axis scales and every test on the geometry from the hanging
+// faces' arithmetic, about a fifth of the instructions of their records, which
+// bound the stage kernels' passes (the vector ALUs are busy 55 % of the FP64
+// kernel, whose passes take 65 % of it, and 71 % of the FP32 one): see the
+// figures at HangStencil.
+enum Cells : int {
+  ANY_CELLS = 0,       // one scale per axis; whether they are powers of two is known at run time
+  DYADIC_CUBES = 1,    // one scale on every axis, a power of two
+  WEIGHTED_CUBES = 2,  // FP64: one scale on every axis, not a power of two (see face_linear's WEIGHTED)
+};
+
 template <class R>
 struct TileGeom {
   R base[3];      // coarsest arm-cell size per axis
@@ -32,9 +44,9 @@ struct TileGeom {
   // its correctly rounded reciprocal
   R wgt, inv_wgt;
   // uniform records decode as UniStencil
-  template <bool WT>
+  template <int CELLS>
   __device__ __forceinline__ bool uni_fast() const {
-    return WT || (pow2 != 0 && cubic != 0);
+    return CELLS != ANY_CELLS || (pow2 != 0 && cubic != 0);
   }
 };
 
@@ -52,25 +64,26 @@ __device__ __forceinline__ uint32_t level_exp(double, uint32_t geo, int f) { ret
 __device__ __forceinline__ float from_exp_bits(float, uint32_t b) { return __uint_as_float(b); }
 __device__ __forceinline__ double from_exp_bits(double, uint32_t b) { return __hiloint2double(int(b), 0); }
 
-template <int D, class R, bool WT = false>
+template <int D, class R, int CELLS = ANY_CELLS>
 __device__ __forceinline__ void decode_dist(uint32_t geo, const TileGeom<R> &g, R *dist, R *q, R *iq) {
   constexpr int F = 2 * D;
-  if (!WT && sizeof(R) == 8 && g.pow2) {
+  constexpr bool ONE = CELLS == DYADIC_CUBES;
+  if (sizeof(R) == 8 && (ONE || (CELLS == ANY_CELLS && g.pow2))) {
     // FP64: base * 2^-l and 2^l / base by exponent arithmetic on the high
     // word (same values, fewer two-word operations); FP32 keeps the
     // multiplications, which measured faster there
 #pragma unroll
     for (int f = 0; f < F; ++f) {
       const uint32_t m = level_exp(R(0), geo, f);
-      q[f] = from_exp_bits(R(0), g.base_bits[f >> 1] - m);
-      iq[f] = from_exp_bits(R(0), g.inv_bits[f >> 1] + m);
+      q[f] = from_exp_bits(R(0), g.base_bits[ONE ? 0 : f >> 1] - m);
+      iq[f] = from_exp_bits(R(0), g.inv_bits[ONE ? 0 : f >> 1] + m);
     }
   } else {
 #pragma unroll
     for (int f = 0; f < F; ++f) {
       const int l = int((geo >> (4 * f)) & 15u);
-      q[f] = g.base[f >> 1] * pow2neg(R(0), l);
-      iq[f] = g.inv_base[f >> 1] * pow2pos(R(0), l);
+      q[f] = g.base[ONE ? 0 : f >> 1] * pow2neg(R(0), l);
+      iq[f] = g.inv_base[ONE ? 0 : f >> 1] * pow2pos(R(0), l);
     }
   }
 #pragma unroll
@@ -88,9 +101,9 @@ __device__ __forceinline__ void decode_dist(uint32_t geo, const TileGeom<R> &g, 
 // wall arm, so every face distance d is a power of two and x / d == x * iq
 // exactly (both are the correctly rounded value of the same real number);
 // FASTDIV lets the stencil arithmetic use that.
-// WT: FP64 on cubic cells whose edge is not a power of two (see face_linear's
-// WEIGHTED); q and dist are base * 2^-l and iq = RN(1 / q) = RN(1 / base) * 2^l.
-template <class R, bool WT>
+// WEIGHTED_CUBES: q and dist are base * 2^-l and iq = RN(1 / q) =
+// RN(1 / base) * 2^l.
+template <class R, bool WEIGHTS>
 struct RegWeight {
   static constexpr bool WEIGHTED = false;
   __device__ __forceinline__ void set_weight(const TileGeom<R> &) {}
@@ -106,8 +119,8 @@ struct RegWeight<R, true> {
   __device__ __forceinline__ R reg_value(R x) const { return weighted_by(x, wgt, inv_wgt); }
 };
 
-template <int D, class R, bool WT = false>
-struct DecodedDist : RegWeight<R, WT> {
+template <int D, class R, int CELLS = ANY_CELLS>
+struct DecodedDist : RegWeight<R, CELLS == WEIGHTED_CUBES> {
   static constexpr bool FASTDIV = true;
   static constexpr bool SLOTS = false;
   static constexpr bool UNIFORM = false;
@@ -118,16 +131,16 @@ struct DecodedDist : RegWeight<R, WT> {
   bool fast, nowall;
   __device__ __forceinline__ R d(int f, int64_t) const { return dist[f]; }
   __device__ __forceinline__ void decode(uint32_t geo, const TileGeom<R> &g) {
-    decode_dist<D, R, WT>(geo, g, dist, q, iq);
+    decode_dist<D, R, CELLS>(geo, g, dist, q, iq);
     nowall = ((geo >> 24) & 63u) == 0u;
-    fast = !WT && g.pow2 && nowall;
+    fast = (CELLS == DYADIC_CUBES || (CELLS == ANY_CELLS && g.pow2)) && nowall;
     this->set_weight(g);
   }
 };
 
 // Stencil of a regular node (no hanging arm): one LDS-local corner per face.
-template <int D, class R, bool WT = false>
-struct RegStencil : DecodedDist<D, R, WT> {
+template <int D, class R, int CELLS = ANY_CELLS>
+struct RegStencil : DecodedDist<D, R, CELLS> {
   static constexpr bool REGULAR = true;
   static constexpr int F = 2 * D;
   uint16_t id[F];
@@ -142,18 +155,18 @@ struct RegStencil : DecodedDist<D, R, WT> {
 };
 
 // Stencil of a uniform node on a geometry of cubic cells (one scale on every
-// axis) that is dyadic (every arm cell a power of two) or WT; the kernels take
+// axis) that is dyadic (every arm cell a power of two) or WEIGHTED; the kernels take
 // this accessor only then, other geometries decode these records as
 // RegStencil: one corner per face, all arms q = base * 2^-level
 // long, no wall.  The per-face arrays hold the same value so the shared
 // stencil code reads them as it reads a RegStencil's.
-template <int D, class R, bool WT = false>
-struct UniStencil : RegWeight<R, WT> {
+template <int D, class R, int CELLS = ANY_CELLS>
+struct UniStencil : RegWeight<R, CELLS == WEIGHTED_CUBES> {
   static constexpr bool REGULAR = true;
   static constexpr bool FASTDIV = true;
   static constexpr bool SLOTS = false;
   static constexpr bool UNIFORM = true;
-  static constexpr bool fast = !WT;
+  static constexpr bool fast = CELLS != WEIGHTED_CUBES;
   static constexpr bool nowall = true;
   static constexpr int F = 2 * D;
   uint16_t id[F];
@@ -214,8 +227,13 @@ struct ExtRegs {
 // for the faces that hang (at most D - 1) the extension record's corners and
 // transverse offsets.  idx / dt serve any face (the per-face functions); the
 // hanging-face functions of stencil_math.hpp use hface / hidx / hdt.
-template <int D, class R, bool WT = false>
-struct HangStencil : DecodedDist<D, R, WT> {
+// CELLS != ANY_CELLS spares the selection of the axis's scale and the six
+// scalings of the transverse extents.  ANY_CELLS and DYADIC_CUBES: 20 stages on
+// 17.5M nodes of a gyroid (FP64, 42 % of the records hang) 14.8 and 13.7 ms, 2
+// advection stages on 8.1M nodes 0.73 and 0.68, 100 stages on 34.2M nodes
+// (mixed, 14 %) 49.6 and 48.1, 512 trees in one launch 2.37 and 2.27.
+template <int D, class R, int CELLS = ANY_CELLS>
+struct HangStencil : DecodedDist<D, R, CELLS> {
   static constexpr bool REGULAR = false;
   static constexpr bool SLOTS = true;
   static constexpr int F = 2 * D, C = 1 << (D - 1);
@@ -227,6 +245,8 @@ struct HangStencil : DecodedDist<D, R, WT> {
   R base[D], inv_base[D];  // the geometry's (uniform values)
   uint64_t d_pack;         // TileGeom::d_pack and lmax
   int lmax;
+  uint32_t base_bits, inv_bits;  // one scale: TileGeom's, and the finest cell
+  R unit;
   // The arm cell size, its inverse and the face distances of the axis of a
   // face f known only at run time, from the level nibbles and wall bits as
   // decode_dist computes them (no indexing of the per-face arrays, which
@@ -243,8 +263,33 @@ struct HangStencil : DecodedDist<D, R, WT> {
     R iqt1, iqt2;     // and their inverses
     R ut1, ut2;       // the finest cell along the transverse axes (offset unit)
   };
+  // base * 2^-l and its inverse, one scale on every axis
+  __device__ __forceinline__ R scaled_down(int l) const {
+    if constexpr (CELLS == DYADIC_CUBES && sizeof(R) == 8) return from_exp_bits(R(0), base_bits - (uint32_t(l) << 20));
+    return base[0] * pow2neg(R(0), l);
+  }
+  __device__ __forceinline__ R scaled_up(int l) const {
+    if constexpr (CELLS == DYADIC_CUBES && sizeof(R) == 8) return from_exp_bits(R(0), inv_bits + (uint32_t(l) << 20));
+    return inv_base[0] * pow2pos(R(0), l);
+  }
   __device__ __forceinline__ SlotGeom slot_geom(int f) const {
     const int a = f >> 1;
+    if constexpr (CELLS != ANY_CELLS) {
+      // one scale: no selection by axis, the transverse extents are the arm cell's size
+      const int le = int((geo >> (8 * a)) & 15u), lo = int((geo >> (8 * a + 4)) & 15u);
+      const R qe = scaled_down(le), qo = scaled_down(lo);
+      const R de = ((geo >> (24 + 2 * a)) & 1u) ? -qo - qe : qe;
+      const R dO = ((geo >> (25 + 2 * a)) & 1u) ? -de - qo : qo;
+      SlotGeom r;
+      r.qf = r.qt1 = r.qt2 = (f & 1) ? qo : qe;
+      r.iqp = scaled_up(lo);
+      r.iqf = r.iqt1 = r.iqt2 = (f & 1) ? r.iqp : scaled_up(le);
+      r.df = (f & 1) ? dO : de;
+      r.dp = dO;
+      r.dm = de;
+      r.ut1 = r.ut2 = unit;
+      return r;
+    }
     R b = base[0], ib = inv_base[0];
 #pragma unroll
     for (int k = 1; k < D; ++k) {
@@ -322,7 +367,7 @@ struct HangStencil : DecodedDist<D, R, WT> {
 #pragma unroll
     for (int f = 0; f < F; ++f) id[f] = rec.idx[f];
     ex = x;
-    pow2 = !WT && g.pow2 != 0;
+    pow2 = CELLS == DYADIC_CUBES || (CELLS == ANY_CELLS && g.pow2 != 0);
     geo = rec.geo;
 #pragma unroll
     for (int k = 0; k < D; ++k) {
@@ -331,6 +376,9 @@ struct HangStencil : DecodedDist<D, R, WT> {
     }
     d_pack = g.d_pack;
     lmax = g.lmax;
+    base_bits = g.base_bits[0];
+    inv_bits = g.inv_bits[0];
+    unit = g.unit[0];
     this->decode(rec.geo, g);
   }
 };
@@ -470,7 +518,7 @@ __device__ __forceinline__ int slot_at(const TileCtx<D> &c, int i, const RecRegs
 // it, the others the general decoding.
 // xrec: the extension record of an irregular position, if the caller already
 // has it in registers.
-template <int D, class R, bool WT = false, bool SMALL = false>
+template <int D, class R, int CELLS = ANY_CELLS, bool SMALL = false>
 __device__ __forceinline__ void tile_pass_a(const TileArgs<R> &A, const TileCtx<D> &c, bool ufast, const RecRegs &r,
                                             int fetched_slot, int i, const R *__restrict__ phis,
                                             R *__restrict__ dds, const ExtRegs<D> *xrec = nullptr) {
@@ -478,17 +526,17 @@ __device__ __forceinline__ void tile_pass_a(const TileArgs<R> &A, const TileCtx<
   R f000, fnb[2 * D], dd[D];
   int j = fetched_slot;
   if (ufast && c.uniform(i)) {
-    UniStencil<D, R, WT> st;
+    UniStencil<D, R, CELLS> st;
     j = st.load(r.w, A.geom);
     laplace<D, R>(st, j, phis, f000, fnb, dd);
   } else {
     const TileRec rec = record_at<D>(c, i, r, j);
     if (!(rec.geo & GEO_IRREGULAR)) {
-      RegStencil<D, R, WT> st;
+      RegStencil<D, R, CELLS> st;
       st.load(rec, A.geom);
       laplace<D, R>(st, j, phis, f000, fnb, dd);
     } else {
-      HangStencil<D, R, WT> st;
+      HangStencil<D, R, CELLS> st;
       if (xrec)
         st.load(rec, *xrec, A.geom);
       else
@@ -547,7 +595,7 @@ constexpr int tile_waves() {
 // arrays phis[LMAX] and dds[D * DMAX].  It reads and writes global memory and
 // the LDS arrays only; a caller running several tiles in a row separates them
 // with a barrier (the next tile overwrites the LDS arrays).
-template <int D, class R, bool SECOND_ORDER, bool RK_AVG, int BLOCK, bool WT = false>
+template <int D, class R, bool SECOND_ORDER, bool RK_AVG, int BLOCK, int CELLS = ANY_CELLS>
 __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__restrict__ phis,
                                            R *__restrict__ dds) {
   constexpr int DMAX = TileLimits<D>::DMAX;
@@ -556,7 +604,7 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
   TileCtx<D> c;
   c.load(A, tile);
   const int s = c.s, nT = c.nT, hb = c.hb, nH = c.nH, nH1 = c.nH1;
-  const bool ufast = A.geom.template uni_fast<WT>();
+  const bool ufast = A.geom.template uni_fast<CELLS>();
   RecRegs trec[KT];
   uint32_t tsf[KT];  // LDS slot of a non-uniform record (low 16 bits) and flags (high 16 bits)
   // the phi_n averaged with in the second RK2 stage: loaded before the first
@@ -636,17 +684,17 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
 #pragma unroll
     for (int k = 0; k < KT; ++k) {
       const int i = int(threadIdx.x) + k * BLOCK;
-      if (i < nT) tile_pass_a<D, R, WT>(A, c, ufast, trec[k], int(tsf[k] & 0xffffu), i, phis, dds);
+      if (i < nT) tile_pass_a<D, R, CELLS>(A, c, ufast, trec[k], int(tsf[k] & 0xffffu), i, phis, dds);
     }
 #pragma unroll
     for (int k = 0; k < K1; ++k) {
       const int i = nT + int(threadIdx.x) + k * BLOCK;
-      if (i < nT + nH1) tile_pass_a<D, R, WT>(A, c, ufast, hrec[k], hslot[k], i, phis, dds);
+      if (i < nT + nH1) tile_pass_a<D, R, CELLS>(A, c, ufast, hrec[k], hslot[k], i, phis, dds);
     }
     for (int i = nT + int(threadIdx.x) + K1 * BLOCK; i < nT + nH1; i += BLOCK) {
       RecRegs r;
       const int js = fetch_record<D>(A, c, i, r);
-      tile_pass_a<D, R, WT>(A, c, ufast, r, js, i, phis, dds);
+      tile_pass_a<D, R, CELLS>(A, c, ufast, r, js, i, phis, dds);
     }
     __syncthreads();
   }
@@ -670,7 +718,7 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
     const int i = int(threadIdx.x) + k * BLOCK;
     if (!(ufast && i < c.nTu)) continue;
     const uint16_t fl = uint16_t(tsf[k] >> 16);
-    using ST = UniStencil<D, R, WT>;
+    using ST = UniStencil<D, R, CELLS>;
     ST st;
     const int j = st.load(trec[k].w, A.geom);
     const R r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, 0, A.sfix + (s + i), A.N,
@@ -687,13 +735,13 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
     const TileRec rec = record_at<D>(c, i, trec[k], j);
     const uint8_t w = uint8_t((rec.geo >> 24) & 63u);
     if (!(rec.geo & GEO_IRREGULAR)) {
-      using ST = RegStencil<D, R, WT>;
+      using ST = RegStencil<D, R, CELLS>;
       ST st;
       st.load(rec, A.geom);
       r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, A.sfix + (s + i), A.N,
                                                                    A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
     } else {
-      using ST = HangStencil<D, R, WT>;
+      using ST = HangStencil<D, R, CELLS>;
       ST st;
       st.load(rec, c.ext_of(A.ext, i), A.geom);
       r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, A.sfix + (s + i), A.N,
@@ -707,7 +755,7 @@ __device__ __forceinline__ void tile_stage(const TileArgs<R> &A, int tile, R *__
 // pass A of phi_0 for T u H1 (second order), then flags and s_fix of the
 // tile's nodes, written in record order (tile start + record position), the
 // order the stage body reads them in.  A.phin is phi_0.
-template <int D, class S, bool SECOND_ORDER, int BLOCK, bool WT = false, bool SMALL = false>
+template <int D, class S, bool SECOND_ORDER, int BLOCK, int CELLS = ANY_CELLS, bool SMALL = false>
 __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, double *__restrict__ phis,
                                           double *__restrict__ dds, const uint8_t *__restrict__ mask,
                                           double lim_low, double lim_high, double zdt,
@@ -716,7 +764,7 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
   TileCtx<D> c;
   c.load(A, tile);
   const int s = c.s, nT = c.nT, hb = c.hb, nH = c.nH, nH1 = c.nH1;
-  const bool ufast = A.geom.template uni_fast<WT>();
+  const bool ufast = A.geom.template uni_fast<CELLS>();
   for (int j = threadIdx.x; j < nT; j += BLOCK) phis[j] = A.phin[s + j];
   for (int j = threadIdx.x; j < nH; j += BLOCK) phis[nT + j] = A.phin[A.halo[hb + j]];
   __syncthreads();
@@ -724,7 +772,7 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
     for (int i = int(threadIdx.x); i < nT + nH1; i += BLOCK) {
       RecRegs r;
       const int js = fetch_record<D>(A, c, i, r);
-      tile_pass_a<D, double, WT, SMALL>(A, c, ufast, r, js, i, phis, dds);
+      tile_pass_a<D, double, CELLS, SMALL>(A, c, ufast, r, js, i, phis, dds);
     }
     __syncthreads();
   }
@@ -733,7 +781,7 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
     int j = fetch_record<D>(A, c, i, r);
     uint16_t fl;
     if (ufast && c.uniform(i)) {
-      using ST = UniStencil<D, double, WT>;
+      using ST = UniStencil<D, double, CELLS>;
       ST st;
       j = st.load(r.w, A.geom);
       const bool masked = mask && mask[s + j] == 0;
@@ -743,13 +791,13 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
       const TileRec rec = record_at<D>(c, i, r, j);
       const bool masked = mask && mask[s + j] == 0;
       if (!(rec.geo & GEO_IRREGULAR)) {
-        using ST = RegStencil<D, double, WT>;
+        using ST = RegStencil<D, double, CELLS>;
         ST st;
         st.load(rec, A.geom);
         fl = prep_value<D, S, ST, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low,
                                                                    lim_high, zdt, SECOND_ORDER, sfix + (s + i), A.N);
       } else {
-        using ST = HangStencil<D, double, WT>;
+        using ST = HangStencil<D, double, CELLS>;
         ST st;
         st.load(rec, c.ext_of(A.ext, i), A.geom);
         fl = prep_value<D, S, ST, SECOND_ORDER>(st, j, masked, phis, dds, DMAX, lim_low,
@@ -761,7 +809,7 @@ __device__ __forceinline__ void tile_prep(const TileArgs<double> &A, int tile, d
   }
 }
 
-template <int D, class S, bool SECOND_ORDER, bool WT = false, bool SMALL = false>
+template <int D, class S, bool SECOND_ORDER, int CELLS = ANY_CELLS, bool SMALL = false>
 __global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
     __attribute__((amdgpu_waves_per_eu((tile_waves<D, double, SMALL>()))))
     k_tile_prep(TileArgs<double> A, const uint8_t *__restrict__ mask, double lim_low, double lim_high, double zdt,
@@ -769,17 +817,17 @@ __global__ void __launch_bounds__((tile_block<D, double, SMALL>()))
   using LIM = TileLimits<D, SMALL>;
   __shared__ double phis[LIM::LMAX];
   __shared__ double dds[SECOND_ORDER ? D * LIM::DMAX : 1];
-  tile_prep<D, S, SECOND_ORDER, tile_block<D, double, SMALL>(), WT, SMALL>(
+  tile_prep<D, S, SECOND_ORDER, tile_block<D, double, SMALL>(), CELLS, SMALL>(
       A, xcd_tile(int(blockIdx.x), int(gridDim.x)), phis, dds, mask, lim_low, lim_high, zdt, flags, sfix);
 }
 
-template <int D, class R, bool SECOND_ORDER, bool RK_AVG, bool WT = false>
+template <int D, class R, bool SECOND_ORDER, bool RK_AVG, int CELLS = ANY_CELLS>
 __global__ void __launch_bounds__((tile_block<D, R, false>()))
     __attribute__((amdgpu_waves_per_eu((tile_waves<D, R, false>()))))
     k_tile_stage(TileArgs<R> A) {
   __shared__ R phis[TileLimits<D>::LMAX];
   __shared__ R dds[SECOND_ORDER ? D * TileLimits<D>::DMAX : 1];
-  tile_stage<D, R, SECOND_ORDER, RK_AVG, tile_block<D, R, false>(), WT>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)),
+  tile_stage<D, R, SECOND_ORDER, RK_AVG, tile_block<D, R, false>(), CELLS>(A, xcd_tile(int(blockIdx.x), int(gridDim.x)),
                                                                        phis, dds);
 }
 
@@ -792,7 +840,7 @@ __global__ void __launch_bounds__((tile_block<D, R, false>()))
 // the halo ids and the phi they name depend on one another.  20 RK2
 // iterations on 14.7K 2D nodes in FP64: 335 us as pass A and pass B kernels,
 // 295 us; 119K 2D nodes mixed, from a graph: 323 and 254 us.
-template <int D, class R, bool SECOND_ORDER, bool RK_AVG, bool WT>
+template <int D, class R, bool SECOND_ORDER, bool RK_AVG, int CELLS>
 __global__ void __launch_bounds__((tile_block<D, R, true>()))
     __attribute__((amdgpu_waves_per_eu((tile_waves<D, R, true>()))))
     k_small_stage(TileArgs<R> A) {
@@ -803,7 +851,7 @@ __global__ void __launch_bounds__((tile_block<D, R, true>()))
   __shared__ R dds[SECOND_ORDER ? D * DMAX : 1];
   TileCtx<D> c;
   c.load(A, xcd_tile(int(blockIdx.x), int(gridDim.x)));
-  const bool ufast = A.geom.template uni_fast<WT>();
+  const bool ufast = A.geom.template uni_fast<CELLS>();
   const int i = int(threadIdx.x), s = c.s;
   const bool own = i < c.nT, active = i < c.nT + (SECOND_ORDER ? c.nH1 : 0);
   constexpr int KH = (LIM::LMAX + BLOCK - 1) / BLOCK;
@@ -837,14 +885,14 @@ __global__ void __launch_bounds__((tile_block<D, R, true>()))
     if (i + k * BLOCK < c.nH) phis[c.nT + i + k * BLOCK] = hv[k];
   __syncthreads();
   if constexpr (SECOND_ORDER) {
-    if (active) tile_pass_a<D, R, WT, true>(A, c, ufast, rec, js, i, phis, dds, &ext);
+    if (active) tile_pass_a<D, R, CELLS, true>(A, c, ufast, rec, js, i, phis, dds, &ext);
     __syncthreads();
   }
   if (!own) return;
   int j = js;
   R r;
   if (ufast && i < c.nTu) {
-    using ST = UniStencil<D, R, WT>;
+    using ST = UniStencil<D, R, CELLS>;
     ST st;
     j = st.load(rec.w, A.geom);
     r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, 0, sf, 1, A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
@@ -852,12 +900,12 @@ __global__ void __launch_bounds__((tile_block<D, R, true>()))
     const TileRec tr = record_at<D>(c, i, rec, j);
     const uint8_t w = uint8_t((tr.geo >> 24) & 63u);
     if (!(tr.geo & GEO_IRREGULAR)) {
-      using ST = RegStencil<D, R, WT>;
+      using ST = RegStencil<D, R, CELLS>;
       ST st;
       st.load(tr, A.geom);
       r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, sf, 1, A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
     } else {
-      using ST = HangStencil<D, R, WT>;
+      using ST = HangStencil<D, R, CELLS>;
       ST st;
       st.load(tr, ext, A.geom);
       r = stage_value<D, R, SECOND_ORDER, ST, true>(st, j, fl, w, sf, 1, A.phi0 + (int64_t(s) + j), phis, dds, DMAX);
@@ -872,5 +920,13 @@ __global__ void __launch_bounds__((tile_block<D, R, true>()))
 // the per-call fields (flags, s_fix, phi_0, phi in and out) are left empty.
 template <class R>
 dev::TileArgs<R> tile_args(const casl_stencil *st);
+
+// The Cells of a stencil's tiles, which run only where use_tiles() says so.
+inline dev::Cells tile_cells(const casl_stencil *st, bool fp64) {
+  if (st->weighted_tiles()) return fp64 ? dev::WEIGHTED_CUBES : dev::ANY_CELLS;
+  bool cubic = true;
+  for (int a = 1; a < st->dim; ++a) cubic = cubic && st->geom_base[a] == st->geom_base[0];
+  return cubic ? dev::DYADIC_CUBES : dev::ANY_CELLS;
+}
 
 }  // namespace casl
