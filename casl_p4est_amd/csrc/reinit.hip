@@ -1144,8 +1144,9 @@ int casl_reinit_graph(casl_stencil_t *st, double *phi, int order_space, int orde
   return guarded([&]() {
     check_reinit_args(st, phi, order_space, order_pseudotime, n_iter, limit_high, limit_low, precision);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // what the recording depends on: the call's arguments, the stage path and
-    // every scratch address the recorded kernels read or write
+    // what the recording depends on: the call's arguments, the kernels that
+    // run them (st->path alone does not say: see use_tiles) and every scratch
+    // address the recorded kernels read or write
     dispatch_reinit(st, phi, nullptr, order_space, order_pseudotime, n_iter, limit_high, limit_low, precision, s,
                     true);
     uint64_t lh, ll;
@@ -1153,7 +1154,8 @@ int casl_reinit_graph(casl_stencil_t *st, double *phi, int order_space, int orde
     std::memcpy(&ll, &limit_low, sizeof(ll));
     const std::vector<uintptr_t> key = {
         uintptr_t(phi), uintptr_t(order_space), uintptr_t(order_pseudotime), uintptr_t(n_iter), uintptr_t(lh),
-        uintptr_t(ll), uintptr_t(precision), uintptr_t(st->path), uintptr_t(st->phi0.p), uintptr_t(st->flags.p),
+        uintptr_t(ll), uintptr_t(precision), uintptr_t(st->use_tiles(precision == CASL_PRECISION_FP64)),
+        uintptr_t(st->phi0.p), uintptr_t(st->flags.p),
         uintptr_t(st->dd0.p), uintptr_t(st->sfix64.p), uintptr_t(st->tmp64.p), uintptr_t(st->ddn64.p),
         uintptr_t(st->sfixf.p), uintptr_t(st->phif.p), uintptr_t(st->tmpf.p), uintptr_t(st->ddnf.p)};
     if (!st->graph_exec || st->graph_key != key) {
