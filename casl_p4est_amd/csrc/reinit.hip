@@ -765,7 +765,7 @@ int casl_stencil_set_path(casl_stencil_t *st, int path) {
 int casl_stencil_get_path(const casl_stencil_t *st, int32_t *path) {
   return guarded([&]() {
     if (!st || !path) throw std::invalid_argument("null argument");
-    *path = st->tiled ? st->path : CASL_PATH_TWO_PASS;
+    *path = st->use_tiles(false) ? CASL_PATH_TILED : CASL_PATH_TWO_PASS;
   });
 }
 

@@ -72,13 +72,15 @@ class DeviceStencil:
 
     def set_path(self, path):
         """"tiled" (fused stage kernel over LDS-staged Morton tiles; the default
-        when the stencil could be tiled) or "two_pass" (grid-wide pass A +
-        pass B)."""
+        when the stencil could be tiled, but for mixed calls on small grids
+        whose cell edges are no powers of two) or "two_pass" (grid-wide pass A
+        + pass B)."""
         code = {"tiled": L.CASL_PATH_TILED, "two_pass": L.CASL_PATH_TWO_PASS}[path]
         L.call("casl_stencil_set_path", self._h, code)
 
     @property
     def path(self):
+        """The path of mixed calls; set_path of it changes no result."""
         v = ctypes.c_int32()
         L.call("casl_stencil_get_path", self._h, ctypes.byref(v))
         return "tiled" if v.value == L.CASL_PATH_TILED else "two_pass"

@@ -96,15 +96,20 @@ int casl_stencil_destroy(casl_stencil_t *st);
 int casl_stencil_info(const casl_stencil_t *st, int32_t *dim, int64_t *n_nodes);
 
 /* Stage kernel selection.  CASL_PATH_TILED: one fused kernel per
- * pseudo-time stage over Morton tiles with LDS-staged halos (the default);
+ * pseudo-time stage over Morton tiles with LDS-staged halos;
  * CASL_PATH_TWO_PASS: grid-wide pass A + pass B kernels.  A stencil without a
- * tiled encoding (cells that are not cubes, or tile limits exceeded;
- * casl_stencil_tile_info gives the reason) runs CASL_PATH_TWO_PASS whatever
- * was set; get_path returns the path that runs.  Two kinds of call run the
- * grid-wide kernels on a tiled stencil: FP64 where the tiles could not give
- * the grid-wide kernels' bits (an origin that rounds the cells' offsets), and
- * mixed calls, unless set_path chose the tiles, on fewer nodes than one
- * full-size tile per compute unit whose cell edges are not powers of two. */
+ * tiled encoding (cells that are not cubes on edges that are not powers of
+ * two, or tile limits exceeded; casl_stencil_tile_info gives the reason) runs
+ * CASL_PATH_TWO_PASS whatever was set.  With one, calls run the tiles unless
+ * set_path chose otherwise, but for two kinds that run the grid-wide kernels:
+ *   - FP64 calls where the tiles could not give the grid-wide kernels' bits (an
+ *     origin that rounds the cells' offsets), whatever was set;
+ *   - mixed calls, unless set_path chose the tiles, on cells whose edges are
+ *     not powers of two where the grid makes fewer full-size tiles than the
+ *     device has compute units (there FP32 rounds differently on the tiles).
+ * get_path returns the path of mixed calls.  Setting the path to what get_path
+ * returned changes no result: where FP64 calls take another path by default
+ * they give the same bits on both. */
 #define CASL_PATH_TILED    0
 #define CASL_PATH_TWO_PASS 1
 int casl_stencil_set_path(casl_stencil_t *st, int path);
