@@ -584,14 +584,17 @@ void upload_tile_host(const TileHost &H, int64_t n_nodes, casl_stencil *st) {
 void upload_tile_tables(const casl_flat_stencil *tab, casl_stencil *st) {
   st->tiled = false;
   TileHost H;
+  int64_t full_tiles = 0;
   try {
     build_tiles(*tab, H, small_tiles(tab->dim, tab->n_nodes));
+    if (!dyadic_scales(H.size, 3)) full_tiles = H.small ? count_tiles(*tab, false) : int64_t(H.tile_start.size()) - 1;
   } catch (const std::exception &e) {
     st->tile_error = e.what();
     return;
   }
   validate_tile_host(H, tab->dim, tab->n_nodes);
   upload_tile_host(H, tab->n_nodes, st);
+  st->full_tiles = full_tiles;
   st->default_path();
 }
 
@@ -706,7 +709,6 @@ void casl_stencil::default_path() {
   hipDeviceProp_t prop;
   HIP_CHECK(hipGetDeviceProperties(&prop, device));
   compute_units = prop.multiProcessorCount;
-  full_tiles = (N + casl::tile_caps(dim, false).tmax - 1) / casl::tile_caps(dim, false).tmax;
   path = CASL_PATH_TILED;
 }
 

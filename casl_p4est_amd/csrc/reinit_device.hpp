@@ -542,16 +542,19 @@ struct casl_stencil {
   // 2.0M-node octree of 64 spheres in [0, 3]^3: 19.6 ms on the grid-wide
   // kernels, 3.03 ms on these.
   //
-  // Mixed calls on a grid of fewer than one full-size tile per compute unit
-  // whose cells are not powers of two stay on the grid-wide kernels unless
-  // the caller picks the tiles: FP32 rounds the weighted form there, the
-  // tiles take the corner's value, and a default call keeps its results.
+  // Mixed calls on a grid that makes fewer full-size tiles than there are
+  // compute units, in cells that are not powers of two, stay on the grid-wide
+  // kernels unless the caller picks the tiles: FP32 rounds the weighted form
+  // there, the tiles take the corner's value, and a default call keeps its
+  // results.
   bool use_tiles(bool fp64) const {
     if (!tiled || path != CASL_PATH_TILED) return false;
     if (dyadic_geometry()) return true;
     return fp64 ? regular_weights : (path_chosen || full_tiles >= compute_units);
   }
-  int64_t full_tiles = 0;  // N over the full-size tile, rounded up
+  // the full-size tiles that the grid makes, halved ones counted, whatever the
+  // size of its tiles (cells that are not powers of two only: see use_tiles)
+  int64_t full_tiles = 0;
   int compute_units = 0;
   // Tiles wherever there is an encoding: one fused kernel per stage against
   // pass A and pass B.  Per RK2 stage (us, FP64 / mixed, two-pass and tiled):

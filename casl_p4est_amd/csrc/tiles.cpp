@@ -359,7 +359,8 @@ struct Builder {
     cut(m, e, out);
   }
 
-  void run(TileHost &H) {
+  // the tiles of every run of caps.tmax nodes
+  std::vector<std::vector<Tile>> cut_all() {
     scan_scales();
     if (!tile_scales_supported(base, D))
       throw std::runtime_error("cells that are not cubes on a box whose edges are not dyadic");
@@ -387,6 +388,11 @@ struct Builder {
       });
     for (auto &th : pool) th.join();
     if (!err.empty()) throw std::runtime_error(err);
+    return parts;
+  }
+
+  void run(TileHost &H) {
+    const std::vector<std::vector<Tile>> parts = cut_all();
     // concatenate
     H.dim = D;
     H.lmax = Lrel;
@@ -431,7 +437,18 @@ struct Builder {
   }
 };
 
+template <int D>
+int64_t count_of(const casl_flat_stencil &tab, bool small) {
+  int64_t n = 0;
+  for (const auto &p : Builder<D>(tab, small).cut_all()) n += int64_t(p.size());
+  return n;
+}
+
 }  // namespace
+
+int64_t count_tiles(const casl_flat_stencil &tab, bool small) {
+  return tab.dim == 2 ? count_of<2>(tab, small) : count_of<3>(tab, small);
+}
 
 void build_tiles(const casl_flat_stencil &tab, TileHost &out, bool small) {
   out.small = small;

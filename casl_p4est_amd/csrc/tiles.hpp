@@ -244,5 +244,7 @@ struct TileHost {
 // used instead).  box sizes are recovered from the arm lengths.  small: cut
 // by the limits of small tiles.
 void build_tiles(const casl_flat_stencil &tab, TileHost &out, bool small);
+// The number of tiles build_tiles would make.
+int64_t count_tiles(const casl_flat_stencil &tab, bool small);
 
 }  // namespace casl

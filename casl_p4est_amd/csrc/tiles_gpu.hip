@@ -857,22 +857,22 @@ struct Round {
   DevBuf<int32_t> counts, halos;
 };
 
+// A tile: its nodes, and where what came of its trial lies.
+struct Tile {
+  int32_t s, e, round, item;
+};
+
+// The tiles of a grid, in order: candidates of the tile size; those whose halo
+// does not fit give way to their halves, which are tried in the next round.
 template <int D, bool SMALL>
-void build_tiles_of(const DTab<D> &tab, const DevBuf<NodeSum> &sum, DevBuf<BuildState> &dstate, BuildState &state,
-                    casl_stencil *st, hipStream_t s) {
+std::vector<Tile> cut_tiles(const DTab<D> &tab, const DevBuf<NodeSum> &sum,
+                            std::vector<std::unique_ptr<Round>> &rounds, hipStream_t s) {
   using B = TileBlock<D, SMALL>;
   using Lim = TileLimits<D, SMALL>;
   const int64_t N = tab.N;
-  const int flags = state.bad;
-  // tiles: candidates of the tile size; those whose halo does not fit give way
-  // to their halves, which are tried in the next round
-  struct Tile {
-    int32_t s, e, round, item;
-  };
   std::vector<Tile> tiles;
   for (int64_t x = 0; x < N; x += Lim::TMAX)
     tiles.push_back({int32_t(x), int32_t(std::min<int64_t>(N, x + Lim::TMAX)), 0, int32_t(tiles.size())});
-  std::vector<std::unique_ptr<Round>> rounds;
   std::vector<TileItem> items;
   for (const Tile &t : tiles) items.push_back({t.s, t.e});
   std::vector<int32_t> counts;
@@ -912,6 +912,18 @@ void build_tiles_of(const DTab<D> &tab, const DevBuf<NodeSum> &sum, DevBuf<Build
     }
     tiles.swap(next);
   }
+  return tiles;
+}
+
+template <int D, bool SMALL>
+void build_tiles_of(const DTab<D> &tab, const DevBuf<NodeSum> &sum, DevBuf<BuildState> &dstate, BuildState &state,
+                    casl_stencil *st, hipStream_t s) {
+  using B = TileBlock<D, SMALL>;
+  using Lim = TileLimits<D, SMALL>;
+  const int64_t N = tab.N;
+  const int flags = state.bad;
+  std::vector<std::unique_ptr<Round>> rounds;
+  const std::vector<Tile> tiles = cut_tiles<D, SMALL>(tab, sum, rounds, s);
   if (flags & BAD_NODE) throw std::runtime_error(bad_reason(BAD_NODE));
 
   // per-tile arrays and record counts
@@ -978,6 +990,11 @@ void build_tiles_of(const DTab<D> &tab, const DevBuf<NodeSum> &sum, DevBuf<Build
   st->tiled = false;
   if (state.bad & ~ODD_WEIGHT) throw std::runtime_error(bad_reason(state.bad));
   st->regular_weights = (state.bad & ODD_WEIGHT) == 0;
+  st->full_tiles = nt;
+  if (SMALL && !st->dyadic_geometry()) {
+    rounds.clear();
+    st->full_tiles = int64_t(cut_tiles<D, false>(tab, sum, rounds, s).size());
+  }
   st->tiled = true;
 }
 
