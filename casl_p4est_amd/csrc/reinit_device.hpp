@@ -540,7 +540,7 @@ struct casl_stencil {
   // grid-wide kernels where the tables do not have that scale exactly (a box
   // origin that rounds the transverse offsets).  20 RK2 iterations on the
   // 2.0M-node octree of 64 spheres in [0, 3]^3: 19.6 ms on the grid-wide
-  // kernels, 3.03 ms on these.
+  // kernels, 3.06 ms on these.
   //
   // Mixed calls on a grid that makes fewer full-size tiles than there are
   // compute units, in cells that are not powers of two, stay on the grid-wide

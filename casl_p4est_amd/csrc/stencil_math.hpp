@@ -229,15 +229,17 @@ template <class R, class TB>
 __device__ __forceinline__ R second_difference(const TB &t, int a, R fp, R f0, R fm, int64_t n) {
   const int fpp = 2 * a + 1, fmm = 2 * a;
   if constexpr (TB::WEIGHTED) {
-    // known reciprocals of the arms; equal arms: d_p + d_m = 2 d_p
-    if (t.nowall) {
-      const R x = (div_known(fp - f0, t.dist[fpp], t.iq[fpp]) + div_known(fm - f0, t.dist[fmm], t.iq[fmm])) * R(2.);
-      if constexpr (TB::UNIFORM) {
-        return div_known(x, R(2.) * t.dist[fpp], R(0.5) * t.iq[fpp]);
-      } else {
-        return t.dist[fpp] == t.dist[fmm] ? div_known(x, R(2.) * t.dist[fpp], R(0.5) * t.iq[fpp])
-                                          : x / (t.dist[fpp] + t.dist[fmm]);
-      }
+    // known reciprocals of the arms; equal arms: d_p + d_m = 2 d_p, and both
+    // factors of 2 drop out
+    if constexpr (TB::UNIFORM) {
+      // infinities, NaN and zeros taken once, from the sum of the differences,
+      // which has the class of the sum of the quotients
+      const R q = t.dist[fpp], iq = t.iq[fpp], a = fp - f0, b = fm - f0;
+      return with_specials(div_number(div_number(a, q, iq) + div_number(b, q, iq), q, iq), a + b, q);
+    } else if (t.nowall) {
+      const R x = div_known(fp - f0, t.dist[fpp], t.iq[fpp]) + div_known(fm - f0, t.dist[fmm], t.iq[fmm]);
+      return t.dist[fpp] == t.dist[fmm] ? div_known(x, t.dist[fpp], t.iq[fpp])
+                                        : x * R(2.) / (t.dist[fpp] + t.dist[fmm]);
     }
     return central_second_derivative(fp, f0, fm, R(t.d(fpp, n)), R(t.d(fmm, n)));
   }

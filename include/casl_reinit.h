@@ -109,7 +109,12 @@ int casl_stencil_info(const casl_stencil_t *st, int32_t *dim, int64_t *n_nodes);
  *     device has compute units (there FP32 rounds differently on the tiles).
  * get_path returns the path of mixed calls.  Setting the path to what get_path
  * returned changes no result: where FP64 calls take another path by default
- * they give the same bits on both. */
+ * they give the same bits on both.
+ * The same bits: for finite phi.  The paths differ in which terms of the form
+ * 0 times an infinity (a NaN) they form.  On cells whose edges are not powers
+ * of two the tiles also need values that are 0 or 1e-250 to 1e250 in magnitude
+ * (their quotients by a cell's length come from its reciprocal); outside, the
+ * last place may differ, or a quotient that overflows be a NaN. */
 #define CASL_PATH_TILED    0
 #define CASL_PATH_TWO_PASS 1
 int casl_stencil_set_path(casl_stencil_t *st, int path);
