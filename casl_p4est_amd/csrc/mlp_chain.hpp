@@ -455,15 +455,16 @@ __global__ void __launch_bounds__(SUM_BLOCK) k_train_sums(SumArgs A) {
     const uint32_t e = blockIdx.x * SUM_BLOCK + t;
     if (e >= A.nw) return;
     float s = A.part[e];
-    int z = 1;
-    for (; z + 21 <= A.splits; z += 21) {  // 63 chunks after the first: three batches of loads
-      float v[21];
+    // sixteen loads in flight ahead of their additions, whatever the number of
+    // chunks (a power of two up to 64: one to four batches after the first)
+    for (int z = 1; z < A.splits; z += 16) {
+      float v[16];
 #pragma unroll
-      for (int k = 0; k < 21; ++k) v[k] = A.part[size_t(z + k) * A.nw + e];
+      for (int k = 0; k < 16; ++k) v[k] = z + k < A.splits ? A.part[size_t(z + k) * A.nw + e] : 0.f;
 #pragma unroll
-      for (int k = 0; k < 21; ++k) s += v[k];
+      for (int k = 0; k < 16; ++k)
+        if (z + k < A.splits) s += v[k];
     }
-    for (; z < A.splits; ++z) s += A.part[size_t(z) * A.nw + e];
     A.gW[e] = s;
     return;
   }
