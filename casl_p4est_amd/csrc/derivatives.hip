@@ -15,6 +15,8 @@
 // else, and first derivatives, run one thread per node on the grid-wide tables.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "reinit_device.hpp"
 #include "tiles_device.hpp"
 
@@ -66,8 +68,11 @@ __global__ void __launch_bounds__(BLOCK) k_curvature(TB t, const double *__restr
 // gradient_central of a tile node from the field in LDS, in the same operation
 // order.  Regular nodes have no correction (their transverse products are 0,
 // so every weight is 0); equal power-of-two arms make every division exact.
-template <int D, class R, class TB>
-__device__ __forceinline__ void tile_gradient(const TB &t, int j, const double *__restrict__ f, double *grad) {
+// tab, n: the grid-wide tables and the node, read for hanging nodes of cells
+// that are not CUBES.
+template <int D, bool CUBES, class TB>
+__device__ __forceinline__ void tile_gradient(const TB &t, int j, const double *__restrict__ f, const Tables<D> &tab,
+                                              int64_t n, double *grad) {
   constexpr int F = 2 * D;
   const double f000 = f[j];
   if constexpr (TB::UNIFORM) {
@@ -85,7 +90,9 @@ __device__ __forceinline__ void tile_gradient(const TB &t, int j, const double *
     for (int a = 0; a < D; ++a)
       grad[a] = central_derivative(fnb[2 * a + 1], f000, fnb[2 * a], t.dist[2 * a + 1], t.dist[2 * a]);
     // the hanging faces' transverse products, and inverse_d_max over arms and
-    // transverse distances (a regular face has its arm cell's size among them)
+    // transverse distances.  In cubes a regular face has its arm cell's size
+    // among them; in other cells its extents are those of the other axes, and
+    // which of them the list holds is known to the tables alone.
     double P[F][2] = {}, m = 0.0;
     const int h0 = t.hface(0), h1 = TB::NH > 1 ? t.hface(TB::NH - 1) : h0;
 #pragma unroll
@@ -110,7 +117,11 @@ __device__ __forceinline__ void tile_gradient(const TB &t, int j, const double *
         }
       }
     }
-    const double idm = 1.0 / m;
+    double idm;
+    if constexpr (CUBES)
+      idm = 1.0 / m;
+    else
+      idm = inverse_d_max<D>(tab, n);
 #pragma unroll
     for (int a = 0; a < D; ++a)
 #pragma unroll
@@ -161,13 +172,13 @@ __device__ __forceinline__ void load_field(const TileArgs<double> &A, const Tile
 
 // compute_normals, one block per tile.  8.4M-node octree: 0.76 ms on the
 // grid-wide tables, 0.17 ms here.
-template <int D>
+template <int D, bool CUBES>
 __global__ void __launch_bounds__(TBLOCK) __attribute__((amdgpu_waves_per_eu(4)))
-    k_tile_normals(TileArgs<double> A, const double *__restrict__ phi, double *__restrict__ nrm) {
+    k_tile_normals(TileArgs<double> A, Tables<D> tab, const double *__restrict__ phi, double *__restrict__ nrm) {
   __shared__ double f[TileLimits<D>::DMAX];
   TileCtx<D> c;
   c.load(A, xcd_tile(int(blockIdx.x), int(gridDim.x)));
-  const bool ufast = A.geom.template uni_fast<false>();
+  const bool ufast = A.geom.template uni_fast<ANY_CELLS>();
   load_field<D>(A, c, phi, f);
   __syncthreads();
   for (int i = int(threadIdx.x); i < c.nT; i += TBLOCK) {
@@ -175,7 +186,7 @@ __global__ void __launch_bounds__(TBLOCK) __attribute__((amdgpu_waves_per_eu(4))
     const int js = fetch_record<D>(A, c, i, r);
     with_record<D>(A, c, ufast, i, r, js, [&](const auto &st, int j) {
       double g[D];
-      tile_gradient<D, double>(st, j, f, g);
+      tile_gradient<D, CUBES>(st, j, f, tab, c.s + j, g);
       double s = g[0] * g[0] + g[1] * g[1];
       if constexpr (D == 3) s = s + g[2] * g[2];
       const double a = sqrt(s);
@@ -187,9 +198,9 @@ __global__ void __launch_bounds__(TBLOCK) __attribute__((amdgpu_waves_per_eu(4))
 
 // One axis of k_tile_curvature: d(n_a)/dx_a added to the partial sums in LDS,
 // or (the last axis) the sum written out.
-template <int D, int AX>
-__device__ __forceinline__ void curvature_axis(const TileArgs<double> &A, const TileCtx<D> &c, bool ufast,
-                                               const double *__restrict__ nrm, double *__restrict__ f,
+template <int D, bool CUBES, int AX>
+__device__ __forceinline__ void curvature_axis(const TileArgs<double> &A, const Tables<D> &tab, const TileCtx<D> &c,
+                                               bool ufast, const double *__restrict__ nrm, double *__restrict__ f,
                                                double *__restrict__ sum, double *__restrict__ kap) {
   load_field<D>(A, c, nrm + int64_t(AX) * A.N, f);
   __syncthreads();
@@ -198,7 +209,7 @@ __device__ __forceinline__ void curvature_axis(const TileArgs<double> &A, const 
     const int js = fetch_record<D>(A, c, i, r);
     with_record<D>(A, c, ufast, i, r, js, [&](const auto &st, int j) {
       double g[D];
-      tile_gradient<D, double>(st, j, f, g);  // the other axes' parts drop out at compile time
+      tile_gradient<D, CUBES>(st, j, f, tab, c.s + j, g);  // the other axes' parts drop out at compile time
       const double k = (AX == 0) ? g[0] : sum[i] + g[AX];
       if constexpr (AX == D - 1)
         kap[c.s + j] = k;
@@ -213,17 +224,17 @@ __device__ __forceinline__ void curvature_axis(const TileArgs<double> &A, const 
 // LDS at a time (the sum over the axes stays in LDS, each thread its own
 // entries: 48 KB, so that blocks share a compute unit).  8.4M-node octree:
 // 1.64 ms on the grid-wide tables, 0.29 ms here.
-template <int D>
+template <int D, bool CUBES>
 __global__ void __launch_bounds__(TBLOCK) __attribute__((amdgpu_waves_per_eu(4)))
-    k_tile_curvature(TileArgs<double> A, const double *__restrict__ nrm, double *__restrict__ kap) {
+    k_tile_curvature(TileArgs<double> A, Tables<D> tab, const double *__restrict__ nrm, double *__restrict__ kap) {
   __shared__ double f[TileLimits<D>::DMAX];
   __shared__ double sum[TileLimits<D>::TMAX];
   TileCtx<D> c;
   c.load(A, xcd_tile(int(blockIdx.x), int(gridDim.x)));
-  const bool ufast = A.geom.template uni_fast<false>();
-  curvature_axis<D, 0>(A, c, ufast, nrm, f, sum, kap);
-  curvature_axis<D, 1>(A, c, ufast, nrm, f, sum, kap);
-  if constexpr (D == 3) curvature_axis<D, 2>(A, c, ufast, nrm, f, sum, kap);
+  const bool ufast = A.geom.template uni_fast<ANY_CELLS>();
+  curvature_axis<D, CUBES, 0>(A, tab, c, ufast, nrm, f, sum, kap);
+  curvature_axis<D, CUBES, 1>(A, tab, c, ufast, nrm, f, sum, kap);
+  if constexpr (D == 3) curvature_axis<D, CUBES, 2>(A, tab, c, ufast, nrm, f, sum, kap);
 }
 
 inline unsigned grid_for(int64_t n) { return unsigned((n + BLOCK - 1) / BLOCK); }
@@ -231,6 +242,15 @@ inline unsigned grid_for(int64_t n) { return unsigned((n + BLOCK - 1) / BLOCK); 
 // The tiles take a call when they are the stencil's path and hold cells of
 // power-of-two edges (the shortcuts above are exact there).
 inline bool on_tiles(const casl_stencil *st) { return st->use_tiles(true) && !st->weighted_tiles(); }
+
+// fn(integral_constant<bool, cubes>) for the tiles of a call on_tiles().
+template <class Fn>
+void with_cubes(const casl_stencil *st, Fn &&fn) {
+  if (tile_cells(st, true) == DYADIC_CUBES)
+    fn(std::true_type{});
+  else
+    fn(std::false_type{});
+}
 
 void check_stencil(const casl_stencil *st, const void *a, const void *b) {
   if (!st || !a || !b) throw std::invalid_argument("null argument");
@@ -262,10 +282,13 @@ int casl_normals(casl_stencil_t *st, const double *phi, double *normals, void *s
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (on_tiles(st)) {
       const dim3 g(unsigned(st->n_tiles)), b(TBLOCK);
-      if (st->dim == 2)
-        hipLaunchKernelGGL(k_tile_normals<2>, g, b, 0, s, tile_args<double>(st), phi, normals);
-      else
-        hipLaunchKernelGGL(k_tile_normals<3>, g, b, 0, s, tile_args<double>(st), phi, normals);
+      with_cubes(st, [&](auto cubes) {
+        constexpr bool CUBES = decltype(cubes)::value;
+        if (st->dim == 2)
+          hipLaunchKernelGGL((k_tile_normals<2, CUBES>), g, b, 0, s, tile_args<double>(st), st->tables<2>(), phi, normals);
+        else
+          hipLaunchKernelGGL((k_tile_normals<3, CUBES>), g, b, 0, s, tile_args<double>(st), st->tables<3>(), phi, normals);
+      });
     } else if (st->dim == 2)
       st->with_tables<2>(true, [&](auto t) {
         hipLaunchKernelGGL((k_normals<2, decltype(t)>), dim3(grid_for(st->N)), dim3(BLOCK), 0, s, t, phi, normals);
@@ -284,10 +307,13 @@ int casl_mean_curvature(casl_stencil_t *st, const double *normals, double *kappa
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (on_tiles(st)) {
       const dim3 g(unsigned(st->n_tiles)), b(TBLOCK);
-      if (st->dim == 2)
-        hipLaunchKernelGGL(k_tile_curvature<2>, g, b, 0, s, tile_args<double>(st), normals, kappa);
-      else
-        hipLaunchKernelGGL(k_tile_curvature<3>, g, b, 0, s, tile_args<double>(st), normals, kappa);
+      with_cubes(st, [&](auto cubes) {
+        constexpr bool CUBES = decltype(cubes)::value;
+        if (st->dim == 2)
+          hipLaunchKernelGGL((k_tile_curvature<2, CUBES>), g, b, 0, s, tile_args<double>(st), st->tables<2>(), normals, kappa);
+        else
+          hipLaunchKernelGGL((k_tile_curvature<3, CUBES>), g, b, 0, s, tile_args<double>(st), st->tables<3>(), normals, kappa);
+      });
     } else if (st->dim == 2)
       st->with_tables<2>(true, [&](auto t) {
         hipLaunchKernelGGL((k_curvature<2, decltype(t)>), dim3(grid_for(st->N)), dim3(BLOCK), 0, s, t, normals, kappa);

@@ -405,9 +405,10 @@ __device__ __forceinline__ int32_t lower_bound_u64(const uint64_t *__restrict__ 
 }
 
 // Ascending keys with the first of every prefix of TOP bits, so that a search
-// spans the keys of one cell of level TOP / D: at most 9 steps where a search
-// of 7.3M leaf keys takes 23.  Every leaf corner looked up: 0.55 ms, 1.18
-// among the 8.1M node keys without the prefixes.
+// spans the keys of one cell of level TOP / D: at most D (finest - TOP / D)
+// steps, 9 on an octree of level 9, where a search of its 7.3M leaf keys takes
+// 23.  Every leaf corner looked up: 0.55 ms, 1.18 among the 8.1M node keys
+// without the prefixes.
 template <int D>
 struct KeyTable {
   static constexpr int TOP = 18, SHIFT = D * Geo<D>::MAXLEVEL - TOP;
