@@ -521,7 +521,7 @@ void chain_backward(casl_mlp *m, const float *x, const float *t, int n, bool wan
 // (the K loop ascends in steps of 16), so the result equals
 // casl_curvature_normalize(_3d) + casl_mlp_forward + casl_curvature_hybrid(_3d)
 // bit for bit.  3.3M samples: 1.36 ms in 3D and 2.26 ms in 2D with activations in
-// LDS and one wave per SIMD, 0.50 and 0.75 ms (890 TFLOP/s) here.
+// LDS and one wave per SIMD, 0.49 and 0.70 ms (710 and 950 TFLOP/s) here.
 struct FusedNet {
   const uint16_t *W16T;  // transposed layers (mlp_chain.hpp)
   const uint16_t *W4;    // the last layer's 128 weights

@@ -13,9 +13,10 @@ namespace dev {
 // What a kernel knows of its tiles' cells when it is compiled.  DYADIC_CUBES
 // drops the per-axis scales and every test on the geometry from the hanging
 // faces' arithmetic, about a fifth of the instructions of their records, which
-// bound the stage kernels' passes (the vector ALUs are busy 55 % of the FP64
-// kernel, whose passes take 65 % of it, and 71 % of the FP32 one): see the
-// figures at HangStencil.
+// bound the stage kernels' passes (the vector ALUs issue for 50 % of the FP64
+// kernel's time on 17.4M nodes of a gyroid and 68 % of the FP32 one's on 34.2M
+// nodes; the passes do not overlap the loads before them): see the figures at
+// HangStencil.
 enum Cells : int {
   ANY_CELLS = 0,       // one scale per axis; whether they are powers of two is known at run time
   DYADIC_CUBES = 1,    // one scale on every axis, a power of two
@@ -849,8 +850,8 @@ __global__ void __launch_bounds__((tile_block<D, R, false>()))
 // can be fetched early is: a record's extension is addressed from its
 // position, the subcell distances from the flags, and only the tile's ranges,
 // the halo ids and the phi they name depend on one another.  20 RK2
-// iterations on 14.7K 2D nodes in FP64: 335 us as pass A and pass B kernels,
-// 295 us; 119K 2D nodes mixed, from a graph: 323 and 254 us.
+// iterations on 14.7K 2D nodes in FP64: 333 us as pass A and pass B kernels,
+// 268 us; 119K 2D nodes mixed, from a graph: 325 and 242 us.
 template <int D, class R, bool SECOND_ORDER, bool RK_AVG, int CELLS>
 __global__ void __launch_bounds__((tile_block<D, R, true>()))
     __attribute__((amdgpu_waves_per_eu((tile_waves<D, R, true>()))))

@@ -351,9 +351,10 @@ int casl_curvature_hybrid(const float *feat, const float *pred, int64_t n,
  * casl_normals) and kappa (from casl_mean_curvature) are FP64 device arrays;
  * feat is [cap][3^dim + 1] FP32.  The samples come in ascending node order.
  * *n_samples may exceed max_samples (then only the first max_samples rows
- * were written); *n_skipped counts band nodes without a uniform block.  The 2D features equal those of
- * kml::Curvature's stencils (my_p4est_curvature_ml.cpp:414-480); the
- * reference has no 3D counterpart. */
+ * were written); *n_skipped counts band nodes without a uniform block.  The
+ * first call allocates 8*dim + 1 bytes a node, which stay with the stencil.
+ * The 2D features equal those of kml::Curvature's stencils
+ * (my_p4est_curvature_ml.cpp:414-480); the reference has no 3D counterpart. */
 int casl_curvature_grid_samples(casl_stencil_t *st, const double *phi,
                                 const double *normals, const double *kappa,
                                 double h, double band, float *feat,
