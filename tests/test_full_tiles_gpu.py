@@ -1,7 +1,8 @@
 """Full-size tiles where the other tests' grids are cut into small ones: FP64
 over cubic cells of an edge that is no power of two, and 2D cells that are not
-cubes, bit for bit as the grid-wide kernels; and a box whose origin rounds the
-offsets of the cells, which stays on the grid-wide kernels in FP64."""
+cubes, bit for bit as the grid-wide kernels, mixed calls within 1e-3 finest
+cells of FP64 near the interface; and a box whose origin rounds the offsets of
+the cells, which stays on the grid-wide kernels in FP64."""
 import ctypes
 
 import numpy as np
@@ -42,6 +43,9 @@ def test_fp64_full_size_tiles(cuda, dim, box, lmin, lmax):
                for space, time in ((2, 2), (2, 1), (1, 2), (1, 1))]
         got.append(ds.reinit(p0.clone(), 2, 2, 3, 0.2 * m, -0.1 * m, 0, mask=mask))
         got.append(ds.advect(p0.clone(), vn, 0.3 * m * 2.0 ** -lmax))
+        mixed = ds.reinit(p0.clone(), 2, 2, 4, C.DBL_MAX, -C.DBL_MAX, 1)
+        h = m * 2.0 ** -lmax
+        assert ds.band_linf(mixed, got[0], got[0], 3 * h) <= 1e-3 * h, path
         out.append(got)
     for k, (a, b) in enumerate(zip(*out)):
         assert torch.equal(a, b), k
